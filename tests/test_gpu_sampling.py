@@ -55,6 +55,30 @@ def test_topk_sample_keeps_every_tie_at_the_kth_value():
             assert torch.equal(ops.topk_sample(logits, noise, k), _torch_draw(logits, noise, k)), k
 
 
+@pytest.mark.parametrize("rows,vocab,k,kind", [
+    (4, 4096, 64, "normal"),      # the largest k of the candidate path
+    (4, 4096, 65, "normal"),      # the first k counted block-wide
+    (3, 8192, 16, "ties"),        # more ties than the candidate list holds
+    (3, 1024, 3, "equal"),        # every logit a candidate, exactly the list's size
+    (3, 1025, 3, "equal"),        # one more than it holds
+    (3, 16384, 16, "masked"),     # fewer finite logits than k: -inf ones are kept with probability 0
+    (2, 63, 16, "normal"),        # waves without any value
+    (2, 32767, 1, "normal"),
+])
+def test_topk_sample_on_both_sides_of_the_candidate_path(rows, vocab, k, kind):
+    g = torch.Generator(device="cuda").manual_seed(vocab + k)
+    for _ in range(4):
+        logits = torch.randn(rows, vocab, device="cuda", generator=g) * 3
+        if kind == "ties":
+            logits = logits.clamp(-1, 1).round()
+        elif kind == "equal":
+            logits = torch.full_like(logits, 0.5)
+        elif kind == "masked":
+            logits[:, 7:] = float("-inf")
+        noise = torch.empty_like(logits).exponential_(1, generator=g)
+        assert torch.equal(ops.topk_sample(logits, noise, k), _torch_draw(logits, noise, k))
+
+
 def test_recorded_sampling_uses_one_launch_and_the_same_noise():
     # the model's draw after a decode step: same tokens as torch.multinomial for the same seed
     g = torch.Generator().manual_seed(8)
