@@ -393,7 +393,7 @@ def time_decode(pkg, cases=DECODE_CASES, iters=50):
         us_app = timed(append, iters)
         app_bytes = b * (hq + 2 * hkv) * d * 4 + b * (hq + 2 * hkv) * d * 2 + d * 4
         res[f"cap{cap}_L{L}"] = {
-            "attention_kernels": "attn_decode_fused_kernel" if fused else "attn_decode_split_kernel + attn_decode_combine_kernel",
+            "attention_kernels": "attn_decode_kernel" if fused else "attn_decode_kernel + attn_decode_combine_kernel",
             "attention_us": round(us, 2), "attention_bytes": attn_bytes,
             "attention_GBps": round(attn_bytes / (us * 1e-6) / 1e9, 1),
             "rope_append_us": round(us_app, 2), "rope_append_bytes": app_bytes}

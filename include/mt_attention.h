@@ -227,6 +227,25 @@ int mt_decode_rope_append(const void* q, const void* k, const void* v, const int
                           void* q_rot, void* k_cache, void* v_cache, const int64_t* cache_strides, int capacity,
                           int B, int Hq, int Hkv, int D, int in_dtype, int dtype, void* stream);
 
+/*
+ * mt_decode_rope_append and the decode attention after it in one launch pair:
+ * the new token's q [B,Hq,D], k/v [B,Hkv,D] (in_strides as above, multiples of
+ * 4 elements for fp32 and 8 for 16-bit inputs) are rounded and rotated as
+ * there, k and v go into the caches at pos, and o [B,Hq,1,D] (contiguous) is
+ * the attention of the rotated q over positions 0 .. length - 1.  The values
+ * are those of the two calls.  pos_dev and length_dev (both or neither) are
+ * read from device memory when the kernels run, clamped to [0, pos] and
+ * [1, capacity].  At most 8 query heads per KV head.  Every pointer 16-byte
+ * aligned.  workspace: mt_gqa_attn_decode_workspace_size(B, Hq, n, D) bytes
+ * with n = capacity for device-length calls, else max(length, pos + 1).
+ */
+int mt_gqa_attn_decode_append(const void* q, const void* k, const void* v, const int64_t* in_strides,
+                              const float* rope_cos, const float* rope_sin, int table_rows, int pos,
+                              const int* pos_dev, void* k_cache, void* v_cache, const int64_t* cache_strides,
+                              int capacity, int length, const int* length_dev, void* o, int B, int Hq, int Hkv, int D,
+                              float scale, int in_dtype, int dtype, void* workspace, size_t workspace_bytes,
+                              void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -214,6 +214,18 @@ def decode_rope_append(query: torch.Tensor, key: torch.Tensor, value: torch.Tens
     ``cos`` / ``sin`` the fp32 RotaryEmbedding tables (row ``pos`` is used).
     ``pos`` is an int or a one-element int32 GPU tensor read when the kernel
     runs (clamped to the cache and table)."""
+    last = _check_append(query, key, value, cos, sin, pos, key_cache, value_cache)
+    # the kernel reads fp32 tables (a model cast with .to(dtype) casts its RoPE buffers too)
+    cos, sin = cos.to(torch.float32), sin.to(torch.float32)
+    if isinstance(pos, torch.Tensor):
+        return torch.ops.mega_trading_amd.decode_rope_append(query, key, value, cos, sin, last, pos, key_cache,
+                                                             value_cache)
+    return torch.ops.mega_trading_amd.decode_rope_append(query, key, value, cos, sin, int(pos), None, key_cache,
+                                                         value_cache)
+
+
+def _check_append(query, key, value, cos, sin, pos, key_cache, value_cache) -> int:
+    """The checks of a decode step's cache append; returns the last valid position."""
     if query.device.type != "cuda":
         raise RuntimeError("hip attention backend requires ROCm GPU tensors")
     for t in (key, value, key_cache, value_cache, cos, sin):
@@ -235,18 +247,49 @@ def decode_rope_append(query: torch.Tensor, key: torch.Tensor, value: torch.Tens
     for name, tab in (("cos", cos), ("sin", sin)):
         if tab.shape[-1] != d // 2 or not tab.is_floating_point():
             raise ValueError(f"RoPE {name} table must be floating point with last dimension head_dim/2 = {d // 2}")
-    # the kernel reads fp32 tables (a model cast with .to(dtype) casts its RoPE buffers too)
-    cos, sin = cos.to(torch.float32), sin.to(torch.float32)
-    last = min(key_cache.shape[2], cos.reshape(-1, cos.shape[-1]).shape[0]) - 1
+    last = min(key_cache.shape[2], cos.numel() // cos.shape[-1]) - 1
     if isinstance(pos, torch.Tensor):
         if pos.dtype != torch.int32 or pos.numel() != 1 or pos.device != query.device:
             raise ValueError("a tensor pos must be a one-element int32 tensor on the query's device")
-        return torch.ops.mega_trading_amd.decode_rope_append(query, key, value, cos, sin, last, pos, key_cache,
-                                                             value_cache)
-    if not 0 <= pos <= last:
+    elif not 0 <= pos <= last:
         raise ValueError(f"pos {pos} outside the cache / RoPE table")
-    return torch.ops.mega_trading_amd.decode_rope_append(query, key, value, cos, sin, int(pos), None, key_cache,
-                                                         value_cache)
+    return last
+
+
+def decode_append_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, cos: torch.Tensor,
+                            sin: torch.Tensor, pos, length, key_cache: torch.Tensor, value_cache: torch.Tensor, *,
+                            repeats: int) -> torch.Tensor:
+    """``decode_rope_append`` then ``decode_attention`` on its rotated query:
+    the same arguments, checks and values.  Where the kernels can load the new
+    rows 16 bytes at a time and a group has at most 8 query heads it is one
+    launch pair (``mt_gqa_attn_decode_append``) instead of two calls."""
+    dev = isinstance(pos, torch.Tensor)
+    b, hq, _, d = query.shape
+    unit = 4 if query.dtype == torch.float32 else 8
+    fused = (query.is_cuda and d in KERNEL_HEAD_DIMS and repeats <= MAX_DECODE_REPEATS
+             and isinstance(length, torch.Tensor) == dev
+             and (dev or 0 <= pos < key_cache.shape[2] and 1 <= length <= key_cache.shape[2])
+             and cos.dtype == torch.float32 and sin.dtype == torch.float32 and cos.is_contiguous() and sin.is_contiguous()
+             and cos.shape == sin.shape
+             and all(t.data_ptr() % 16 == 0 for t in (query, key, value, cos, sin, key_cache, value_cache))
+             and all(st % unit == 0 for t in (query, key, value) for st in t.stride()[:2])
+             and all(st % 8 == 0 for t in (key_cache, value_cache) for st in t.stride()[:3]))
+    if not fused:
+        q_rot = decode_rope_append(query, key, value, cos, sin, pos, key_cache, value_cache)
+        return decode_attention(q_rot, key_cache, value_cache, length, repeats=repeats)
+    last = _check_append(query, key, value, cos, sin, pos, key_cache, value_cache)
+    if query.shape[2] != 1 or key.shape != (b, key_cache.shape[1], 1, d) or value.shape != key.shape:
+        raise ValueError("query must be [B, Hq, 1, D] and key / value [B, Hkv, 1, D] with the caches' B and Hkv")
+    if key_cache.shape[1] * repeats != hq or key_cache.shape[0] != b:
+        raise ValueError("query heads must equal key/value heads multiplied by repeats")
+    scale = 1.0 / math.sqrt(d)
+    if dev:
+        if length.dtype != torch.int32 or length.numel() != 1 or length.device != query.device:
+            raise ValueError("a tensor length must be a one-element int32 tensor on the query's device")
+        return torch.ops.mega_trading_amd.gqa_attn_decode_append(query, key, value, cos, sin, last, pos, 0, length,
+                                                                 key_cache, value_cache, scale)
+    return torch.ops.mega_trading_amd.gqa_attn_decode_append(query, key, value, cos, sin, int(pos), None, int(length),
+                                                             None, key_cache, value_cache, scale)
 
 
 # ---------------------------------------------------------------------------
@@ -478,6 +521,37 @@ def gqa_attn_decode_dev(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.T
                                         ws.data_ptr(), ws_bytes, torch.cuda.current_stream(q.device).cuda_stream)
     _native.check(rc, "mt_gqa_attn_decode_dev")
     return out
+
+
+@torch.library.custom_op("mega_trading_amd::gqa_attn_decode_append", mutates_args=("k_cache", "v_cache"),
+                         device_types="cuda")
+def gqa_attn_decode_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+                           pos: int, pos_dev: Optional[torch.Tensor], length: int, length_dev: Optional[torch.Tensor],
+                           k_cache: torch.Tensor, v_cache: torch.Tensor, scale: float) -> torch.Tensor:
+    import ctypes
+
+    lib = _native.load()
+    b, hq, _, d = q.shape
+    hkv, cap = k_cache.shape[1], k_cache.shape[2]
+    out = torch.empty((b, hq, 1, d), device=q.device, dtype=k_cache.dtype)
+    ins = (ctypes.c_int64 * 6)(q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1))
+    cst = (ctypes.c_int64 * 6)(*k_cache.stride()[:3], *v_cache.stride()[:3])
+    in_dt = _native.DTYPE_FP32 if q.dtype == torch.float32 else _KERNEL_DTYPES[q.dtype]
+    with torch.cuda.device(q.device):
+        ws_bytes = lib.mt_gqa_attn_decode_workspace_size(b, hq, cap if length_dev is not None else max(length, pos + 1), d)
+        ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)
+        rc = lib.mt_gqa_attn_decode_append(q.data_ptr(), k.data_ptr(), v.data_ptr(), ins, cos.data_ptr(), sin.data_ptr(),
+                                           cos.numel() // (d // 2), pos, _ptr(pos_dev), k_cache.data_ptr(),
+                                           v_cache.data_ptr(), cst, cap, length, _ptr(length_dev), out.data_ptr(), b, hq,
+                                           hkv, d, scale, in_dt, _KERNEL_DTYPES[k_cache.dtype], ws.data_ptr(), ws_bytes,
+                                           torch.cuda.current_stream(q.device).cuda_stream)
+    _native.check(rc, "mt_gqa_attn_decode_append")
+    return out
+
+
+@gqa_attn_decode_append.register_fake
+def _gqa_attn_decode_append_fake(q, k, v, cos, sin, pos, pos_dev, length, length_dev, k_cache, v_cache, scale):
+    return q.new_empty(q.shape, dtype=k_cache.dtype)
 
 
 @gqa_attn_decode_dev.register_fake

@@ -679,27 +679,61 @@ int mt_gqa_attn_bwd_dkv(MT_BWD_ARGS) { return bwd_impl(2, MT_BWD_PASS); }
 
 size_t mt_gqa_attn_decode_workspace_size(int B, int Hq, int L, int D) {
   if (B < 1 || Hq < 1 || L < 1 || D < 1) return 0;
-  const size_t nsplit = (size_t)((L + mt::kDecSplit - 1) / mt::kDecSplit);
-  return ((size_t)B * Hq * nsplit * (D + 4) * sizeof(float) + 255) / 256 * 256;  // rows of mt::dec_row<D>()
+  const int span = mt::kDecSplit * mt::kDecMinWaves;  // the smallest keys per workgroup: the most partials
+  const size_t nspan = (size_t)((L + span - 1) / span);
+  return ((size_t)B * Hq * nspan * (D + 4) * sizeof(float) + 255) / 256 * 256;  // rows of mt::dec_row<D>()
 }
 
 namespace {
 
-// A cache of at most kDecWaves splits of 64 keys (its capacity, for
-// device-length launches) is decoded by the fused kernel, one workgroup per
-// (batch, KV head); longer caches by the split + combine pair, whose grid
-// grows with the length.
+// Waves (of 64 keys) per workgroup, L the capacity for device-length launches.
+// 512 keys are one workgroup of 8 waves and one launch.  1024 keys of D <= 64
+// are one of 16 waves where there are enough (batch, KV head) pairs to spread
+// over the CUs (8 / 2 heads of 64, bf16, us: 128 pairs 8.6 against 11.4 for 4
+// waves and the merge launch at L = 700, 64 pairs 7.8 against 8.1 at L = 545;
+// 16 pairs 9.0 against 7.5 at L = 1000, a workgroup's keys come through one
+// CU's 64 B/clk).  Everything longer takes 4 waves: 8 are 3 % faster for 94
+// splits of 32 / 8 heads of 128 but 30 % slower at 7 heads a group (the merge
+// and the registers of the longer workgroup hide less of the loads).
+int decode_waves(int64_t pairs, int L, int D) { return L <= 512 ? 8 : L <= 1024 && D <= 64 && pairs >= 64 ? 16 : 4; }
+
 extern "C++" {
 template <class E, int D, int R>
-void launch_decode(const mt::DecodeParams& p, dim3 grid_f, dim3 grid_s, dim3 grid_c, hipStream_t st) {
-  if (p.nsplit <= mt::kDecWaves) {
-    hipLaunchKernelGGL((mt::attn_decode_fused_kernel<E, D, R>), grid_f, dim3(64 * mt::kDecWaves), 0, st, p);
-    return;
-  }
-  hipLaunchKernelGGL((mt::attn_decode_split_kernel<E, D, R>), grid_s, dim3(64), 0, st, p);
-  hipLaunchKernelGGL((mt::attn_decode_combine_kernel<E, D>), grid_c, dim3(256), 0, st, p);
+void launch_decode(const mt::DecodeParams& p, hipStream_t st) {
+  const dim3 grid((unsigned)(p.B * p.Hkv * p.nspan));
+  if (p.span == 16 * mt::kDecSplit) {
+    if constexpr (D <= 64) hipLaunchKernelGGL((mt::attn_decode_kernel<E, D, R, 16>), grid, dim3(64 * 16), 0, st, p);
+  } else if (p.span == 8 * mt::kDecSplit)
+    hipLaunchKernelGGL((mt::attn_decode_kernel<E, D, R, 8>), grid, dim3(64 * 8), 0, st, p);
+  else
+    hipLaunchKernelGGL((mt::attn_decode_kernel<E, D, R, 4>), grid, dim3(64 * 4), 0, st, p);
+  if (p.nspan > 1)
+    hipLaunchKernelGGL((mt::attn_decode_combine_kernel<E, D>), dim3((unsigned)(((int64_t)p.B * p.Hq * D + 255) / 256)),
+                       dim3(256), 0, st, p);
 }
 }  // extern "C++"
+
+int run_decode(const mt::DecodeParams& p, int D, int dtype, void* stream) {
+  hipStream_t st = (hipStream_t)stream;
+  // the decode kernels are instantiated per group size R = Hq / Hkv (1..8)
+#define MT_DECODE_SPLIT(E, DD, RR) \
+  case RR: launch_decode<E, DD, RR>(p, st); break
+#define MT_DECODE_LAUNCH(E, DD)                                                                            \
+  switch (p.R) {                                                                                           \
+    MT_DECODE_SPLIT(E, DD, 1); MT_DECODE_SPLIT(E, DD, 2); MT_DECODE_SPLIT(E, DD, 3); MT_DECODE_SPLIT(E, DD, 4); \
+    MT_DECODE_SPLIT(E, DD, 5); MT_DECODE_SPLIT(E, DD, 6); MT_DECODE_SPLIT(E, DD, 7); MT_DECODE_SPLIT(E, DD, 8); \
+    default: break;                                                                                        \
+  }
+  if (dtype == MT_DTYPE_BF16) {
+    if (D == 32) { MT_DECODE_LAUNCH(mt::BF16, 32); } else if (D == 64) { MT_DECODE_LAUNCH(mt::BF16, 64); } else { MT_DECODE_LAUNCH(mt::BF16, 128); }
+  } else {
+    if (D == 32) { MT_DECODE_LAUNCH(mt::FP16, 32); } else if (D == 64) { MT_DECODE_LAUNCH(mt::FP16, 64); } else { MT_DECODE_LAUNCH(mt::FP16, 128); }
+  }
+#undef MT_DECODE_SPLIT
+#undef MT_DECODE_LAUNCH
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? ok() : fail((int)e, "decode launch failed: %s", hipGetErrorString(e));
+}
 
 int decode_impl(const void* q, const void* k_cache, const void* v_cache, void* o, int B, int Hq, int Hkv, int L,
                 const int* length_dev, int D, const int64_t* strides, float scale, int dtype, void* workspace,
@@ -730,30 +764,10 @@ int decode_impl(const void* q, const void* k_cache, const void* v_cache, void* o
   p.so[0] = strides[12]; p.so[1] = strides[13];
   p.length_dev = length_dev;
   p.B = B; p.Hq = Hq; p.Hkv = Hkv; p.R = Hq / Hkv; p.L = L;
-  p.nsplit = (L + mt::kDecSplit - 1) / mt::kDecSplit;
+  p.span = decode_waves((int64_t)B * Hkv, L, D) * mt::kDecSplit;
+  p.nspan = (L + p.span - 1) / p.span;
   p.scale_log2 = scale * mt::kLog2e;
-  hipStream_t st = (hipStream_t)stream;
-  const dim3 grid_f((unsigned)(B * Hkv));
-  const dim3 grid_s((unsigned)(B * Hkv * p.nsplit));
-  const dim3 grid_c((unsigned)(((int64_t)B * Hq * D + 255) / 256));
-  // the decode kernels are instantiated per group size R = Hq / Hkv (1..8)
-#define MT_DECODE_SPLIT(E, DD, RR) \
-  case RR: launch_decode<E, DD, RR>(p, grid_f, grid_s, grid_c, st); break
-#define MT_DECODE_LAUNCH(E, DD)                                                                            \
-  switch (p.R) {                                                                                           \
-    MT_DECODE_SPLIT(E, DD, 1); MT_DECODE_SPLIT(E, DD, 2); MT_DECODE_SPLIT(E, DD, 3); MT_DECODE_SPLIT(E, DD, 4); \
-    MT_DECODE_SPLIT(E, DD, 5); MT_DECODE_SPLIT(E, DD, 6); MT_DECODE_SPLIT(E, DD, 7); MT_DECODE_SPLIT(E, DD, 8); \
-    default: break;                                                                                        \
-  }
-  if (dtype == MT_DTYPE_BF16) {
-    if (D == 32) { MT_DECODE_LAUNCH(mt::BF16, 32); } else if (D == 64) { MT_DECODE_LAUNCH(mt::BF16, 64); } else { MT_DECODE_LAUNCH(mt::BF16, 128); }
-  } else {
-    if (D == 32) { MT_DECODE_LAUNCH(mt::FP16, 32); } else if (D == 64) { MT_DECODE_LAUNCH(mt::FP16, 64); } else { MT_DECODE_LAUNCH(mt::FP16, 128); }
-  }
-#undef MT_DECODE_SPLIT
-#undef MT_DECODE_LAUNCH
-  const hipError_t e = hipGetLastError();
-  return e == hipSuccess ? ok() : fail((int)e, "decode launch failed: %s", hipGetErrorString(e));
+  return run_decode(p, D, dtype, stream);
 }
 
 }  // namespace
@@ -771,6 +785,64 @@ int mt_gqa_attn_decode_dev(const void* q, const void* k_cache, const void* v_cac
   if (!length_dev) return fail(MT_E_NULL, "length_dev is NULL");
   return decode_impl(q, k_cache, v_cache, o, B, Hq, Hkv, capacity, length_dev, D, strides, scale, dtype, workspace,
                      workspace_bytes, stream);
+}
+
+int mt_gqa_attn_decode_append(const void* q, const void* k, const void* v, const int64_t* in_strides,
+                              const float* rope_cos, const float* rope_sin, int table_rows, int pos,
+                              const int* pos_dev, void* k_cache, void* v_cache, const int64_t* cache_strides,
+                              int capacity, int length, const int* length_dev, void* o, int B, int Hq, int Hkv, int D,
+                              float scale, int in_dtype, int dtype, void* workspace, size_t workspace_bytes,
+                              void* stream) {
+  int rc = check_common(B, Hq, Hkv, capacity, D, dtype, rope_cos, rope_sin);
+  if (rc) return rc;
+  if (dtype == MT_DTYPE_FP32) return fail(MT_E_DTYPE, "the KV caches must be bfloat16 or float16");
+  if (in_dtype != MT_DTYPE_FP32 && in_dtype != dtype)
+    return fail(MT_E_DTYPE, "inputs must be float32 or have the cache dtype (got code %d)", in_dtype);
+  if (Hq / Hkv > mt::kDecMaxR)
+    return fail(MT_E_SHAPE, "decode supports up to %d query heads per KV head (got %d)", mt::kDecMaxR, Hq / Hkv);
+  if (!q || !k || !v || !k_cache || !v_cache || !o || !rope_cos || !rope_sin || !in_strides || !cache_strides || !workspace)
+    return fail(MT_E_NULL, "q, k, v, the caches, o, the rope tables, strides and workspace must be non-NULL");
+  if (table_rows < 1) return fail(MT_E_SHAPE, "RoPE table rows must be >= 1 (got %d)", table_rows);
+  if (pos < 0 || pos >= capacity || pos >= table_rows)
+    return fail(MT_E_SHAPE, "pos %d outside the cache (capacity %d) or the RoPE table (%d rows)", pos, capacity,
+                table_rows);
+  if ((length_dev == nullptr) != (pos_dev == nullptr))
+    return fail(MT_E_NULL, "pos_dev and length_dev must be given together");
+  if (!length_dev && (length < 1 || length > capacity))
+    return fail(MT_E_SHAPE, "length %d outside [1, capacity %d]", length, capacity);
+  // 16-byte loads and stores of every row
+  const int unit = in_dtype == MT_DTYPE_FP32 ? 4 : 8;
+  for (int i = 0; i < 6; ++i) {
+    if (in_strides[i] % unit) return fail(MT_E_STRIDE, "input strides must be multiples of %d", unit);
+    if (cache_strides[i] % 8) return fail(MT_E_STRIDE, "cache strides must be multiples of 8");
+  }
+  const void* ptrs[9] = {q, k, v, k_cache, v_cache, o, rope_cos, rope_sin, workspace};
+  for (const void* x : ptrs)
+    if (reinterpret_cast<uintptr_t>(x) % 16) return fail(MT_E_STRIDE, "every pointer must be 16-byte aligned");
+  const int cover = length_dev ? capacity : (length > pos ? length : pos + 1);  // keys read, and the row written
+  if (workspace_bytes < mt_gqa_attn_decode_workspace_size(B, Hq, cover, D))
+    return fail(MT_E_WORKSPACE, "workspace of %zu bytes is smaller than the %zu required", workspace_bytes,
+                mt_gqa_attn_decode_workspace_size(B, Hq, cover, D));
+  mt::DecodeParams p{};
+  p.xq = q; p.xk = k; p.xv = v;
+  for (int i = 0; i < 2; ++i) {
+    p.sxq[i] = in_strides[i]; p.sxk[i] = in_strides[2 + i]; p.sxv[i] = in_strides[4 + i];
+  }
+  for (int i = 0; i < 3; ++i) { p.sk[i] = cache_strides[i]; p.sv[i] = cache_strides[3 + i]; }
+  p.k = p.kc = static_cast<uint16_t*>(k_cache);
+  p.v = p.vc = static_cast<uint16_t*>(v_cache);
+  p.out = static_cast<uint16_t*>(o);
+  p.part = static_cast<float*>(workspace);
+  p.so[0] = (int64_t)Hq * D; p.so[1] = D;
+  p.cos = rope_cos; p.sin = rope_sin;
+  p.pos = pos; p.pos_dev = pos_dev; p.length_dev = length_dev;
+  p.in_fp32 = in_dtype == MT_DTYPE_FP32;
+  p.B = B; p.Hq = Hq; p.Hkv = Hkv; p.R = Hq / Hkv;
+  p.L = length_dev ? capacity : length;
+  p.span = decode_waves((int64_t)B * Hkv, cover, D) * mt::kDecSplit;
+  p.nspan = (cover + p.span - 1) / p.span;
+  p.scale_log2 = scale * mt::kLog2e;
+  return run_decode(p, D, dtype, stream);
 }
 
 int mt_decode_rope_append(const void* q, const void* k, const void* v, const int64_t* in_strides,

@@ -43,8 +43,7 @@ from torch import nn
 from . import _native
 from .attention import KERNEL_HEAD_DIMS, _rope_tables
 from .attention import attention as _hip_attention
-from .attention import decode_attention as _hip_decode_attention
-from .attention import decode_rope_append as _hip_decode_rope_append
+from .attention import decode_append_attention as _hip_decode_append_attention
 from .attention import rope_attention as _hip_rope_attention
 from .attention import rope_attention_packed as _hip_rope_attention_packed
 from .ops import fused_linear_cross_entropy as _hip_fused_linear_cross_entropy
@@ -454,9 +453,9 @@ class LlamaAttention(nn.Module):
         the caches, attend over positions 0..pos."""
         b, _, hidden_dim = hidden.shape
         query, key, value = self._heads(hidden)
-        q_rot = _hip_decode_rope_append(query, key, value, self.rope.cos, self.rope.sin, pos, k_cache, v_cache)
-        out = _hip_decode_attention(q_rot, k_cache, v_cache, pos + 1 if length is None else length,
-                                    repeats=self.repeats)
+        out = _hip_decode_append_attention(query, key, value, self.rope.cos, self.rope.sin, pos,
+                                           pos + 1 if length is None else length, k_cache, v_cache,
+                                           repeats=self.repeats)
         if self.attention_backend != "hip":
             out = out.to(hidden.dtype)
         # on "hip" o_proj takes the 16-bit output as it is (the few-row product

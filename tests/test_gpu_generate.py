@@ -357,3 +357,32 @@ def test_recorded_decode_with_a_large_vocabulary_samples_like_the_eager_step():
         recorded = m.generate(prompt, max_new_tokens=24, top_k=16)
         torch.cuda.synchronize()
         assert torch.equal(recorded, eager)
+
+
+@pytest.mark.parametrize("b,hq,hkv,d,cap,pos,in_dt,dev", [
+    (3, 8, 2, 64, 40, 17, torch.float32, False),
+    (2, 8, 2, 64, 512, 511, torch.float32, True),      # the last position of one 8-wave workgroup
+    (2, 6, 2, 32, 513, 512, torch.bfloat16, True),     # the first of a second workgroup
+    (33, 4, 2, 64, 1024, 1023, torch.float32, True),   # 66 (batch, KV head) pairs: one 16-wave workgroup
+    (32, 4, 2, 64, 1025, 1024, torch.float32, False),  # 4-wave workgroups and the merge
+    (2, 7, 1, 128, 300, 64, torch.float16, True),
+    (1, 8, 1, 128, 2048, 63, torch.float32, False),
+    (2, 9, 1, 64, 128, 5, torch.float32, False),       # a group of 9 heads: the two calls
+])
+def test_decode_append_attention_equals_the_two_calls(b, hq, hkv, d, cap, pos, in_dt, dev):
+    attn = importlib.import_module("mega-trading_amd.attention")
+    dt = torch.float16 if in_dt == torch.float16 else torch.bfloat16
+    g = torch.Generator().manual_seed(cap + pos)
+    qkv = torch.randn(b, 1, (hq + 2 * hkv) * d, generator=g).to(in_dt).cuda()  # a packed projection
+    q, k, v = (t.view(b, 1, -1, d).transpose(1, 2) for t in qkv.split([hq * d, hkv * d, hkv * d], dim=-1))
+    rope = model_mod.RotaryEmbedding(d, cap, theta=10_000.0).cuda()
+    kc, vc = (torch.randn(b, hkv, cap, d, generator=g).to(dt).cuda() for _ in range(2))
+    at = torch.tensor([pos], dtype=torch.int32, device="cuda") if dev else pos
+    for length in {pos + 1, max(1, pos // 2), min(cap, pos + 70)}:  # also lengths that are not pos + 1
+        n = torch.tensor([length], dtype=torch.int32, device="cuda") if dev else length
+        k1, v1, k2, v2 = kc.clone(), vc.clone(), kc.clone(), vc.clone()
+        k2[:, :, pos] = float("nan")  # the stale row is never used
+        ref = attn.decode_attention(attn.decode_rope_append(q, k, v, rope.cos, rope.sin, at, k1, v1), k1, v1, n,
+                                    repeats=hq // hkv)
+        got = attn.decode_append_attention(q, k, v, rope.cos, rope.sin, at, n, k2, v2, repeats=hq // hkv)
+        assert torch.equal(k1, k2) and torch.equal(v1, v2) and torch.equal(ref, got), length
