@@ -187,6 +187,16 @@ int mt_linear_rows(const void* x, int64_t x_row_stride, const void* const* weigh
                    const int64_t* w_row_strides, int groups, void* y, int64_t y_row_stride, int rows, int in_features,
                    int dtype, void* stream);
 
+/*
+ * The gate of a SwiGLU over two such products without writing them:
+ * y[m, n] = silu(g) * u, g = sum_k x[m, k] w_gate[n, k], u the same with w_up,
+ * n < out_features; fp32, the values of mt_linear_rows followed by
+ * mt_swiglu_packed_fwd.  Arguments as there.
+ */
+int mt_linear_rows_gate(const void* x, int64_t x_row_stride, const void* w_gate, const void* w_up,
+                        int64_t gate_row_stride, int64_t up_row_stride, void* y, int64_t y_row_stride, int rows,
+                        int in_features, int out_features, int dtype, void* stream);
+
 /* One sampled token per row: the logits >= the k-th largest of the row are
  * kept (ties at the k-th value included), p = softmax over the kept values,
  * and tokens[r] = the first index of the largest p / E[r, i] over the kept i,

@@ -54,6 +54,7 @@ EXPORTS = (
     "mt_decode_rope_append",
     "mt_gqa_attn_decode_append",
     "mt_linear_rows",
+    "mt_linear_rows_gate",
     "mt_topk_sample",
 )
 
@@ -93,6 +94,7 @@ _OPS_SIGNATURES = {
     "mt_gqa_attn_decode_append": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _P, _P, _P, _P, _I, _I, _P, _P, _I, _I, _I, _I,
                                        _F, _I, _I, _P, _S, _P]),
     "mt_linear_rows": (_I, [_P, _L, _P, _P, _P, _I, _P, _L, _I, _I, _I, _P]),
+    "mt_linear_rows_gate": (_I, [_P, _L, _P, _P, _L, _L, _P, _L, _I, _I, _I, _I, _P]),
     "mt_topk_sample": (_I, [_P, _L, _P, _L, _I, _I, _I, _P, _I, _P]),
 }
 

@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "mt_common.h"
+#include "ops_kernels.h"
 
 namespace mt {
 
@@ -63,21 +64,31 @@ __device__ __forceinline__ f32x4 load_x4(const void* row, int k) {
 
 // PD: chunks of 4 values per lane held in flight (all of them when K <= 128 PD).
 // XT: float, or BF16 / FP16 for a 16-bit x.
-template <int PD, class XT>
+// GATE: groups 0 and 1 are the gate and up projections of a SwiGLU, equally
+// wide: a workgroup forms both 16 x 16 tiles from one read of x and writes
+// silu(gate) * up [M, n] (the values of the two products followed by the gate
+// kernel), so the packed product is neither written nor read back and the gate
+// costs no launch.  Measured at 32 rows, 512 -> 2 x 1408 (kernel trace): product
+// 7.5 us and gate kernel 2.8 us before, 5.5 us together.
+template <int PD, class XT, bool GATE>
 __global__ __launch_bounds__(64 * kLinWaves) void linear_rows_f32_kernel(LinearParams p) {
-  __shared__ float red[kLinWaves][16][17];
+  constexpr int T = GATE ? 2 : 1;  // weight tiles per workgroup
+  __shared__ float red[T][kLinWaves][16][17];
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
   const int lane = tid & 63;
   const int q = lane >> 4;   // contraction slot
   const int c = lane & 15;   // A row / B column of this lane
-  const int ntiles = p.g[p.groups - 1].tile0 + (p.g[p.groups - 1].n + kLinCols - 1) / kLinCols;
+  const int last = GATE ? 0 : p.groups - 1;
+  const int ntiles = p.g[last].tile0 + (p.g[last].n + kLinCols - 1) / kLinCols;
   const int ct = (int)blockIdx.x % ntiles;  // column tile
   const int m0 = ((int)blockIdx.x / ntiles) * 16;
   int gi = 0;
+  if constexpr (!GATE) {
 #pragma unroll
-  for (int i = 1; i < kLinGroups; ++i)
-    if (i < p.groups && ct >= p.g[i].tile0) gi = i;
+    for (int i = 1; i < kLinGroups; ++i)
+      if (i < p.groups && ct >= p.g[i].tile0) gi = i;
+  }
   const LinearGroup grp = p.g[gi];
   const int n0 = (ct - grp.tile0) * kLinCols;
 
@@ -85,15 +96,21 @@ __global__ __launch_bounds__(64 * kLinWaves) void linear_rows_f32_kernel(LinearP
   // those lane quarter q the 16-byte blocks 4 j + q (j = 0 .. K / 128 - 1), so
   // for each j the four quarters of a row read 64 contiguous bytes
   const int k0 = wave * (p.K >> 3) + 4 * q;
-  const float* wrow = grp.w + (int64_t)min(n0 + c, grp.n - 1) * grp.ldw + k0;
+  const float* wrow[T];
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+    wrow[t] = p.g[gi + t].w + (int64_t)min(n0 + c, grp.n - 1) * p.g[gi + t].ldw + k0;
   constexpr int XB = std::is_same_v<XT, float> ? 4 : 2;  // bytes per x value
   const void* xrow = static_cast<const char*>(p.x) + ((int64_t)min(m0 + c, p.M - 1) * p.ldx + k0) * XB;
 
-  f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // two chains: back-to-back issue
+  f32x4 acc[T][2];  // two chains: back-to-back issue
+#pragma unroll
+  for (int t = 0; t < T; ++t) acc[t][0] = acc[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int nch = p.K >> 7;
-  f32x4 wb[PD], xb[PD];
+  f32x4 wb[T][PD], xb[PD];
   auto load = [&](int j, int kk) {
-    wb[j] = *reinterpret_cast<const f32x4*>(wrow + kk);
+#pragma unroll
+    for (int t = 0; t < T; ++t) wb[t][j] = *reinterpret_cast<const f32x4*>(wrow[t] + kk);
     xb[j] = load_x4<XT>(xrow, kk);
   };
 #pragma unroll
@@ -106,22 +123,34 @@ __global__ __launch_bounds__(64 * kLinWaves) void linear_rows_f32_kernel(LinearP
       if (i < nch) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          acc[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(xb[j][e], wb[j][e], acc[e & 1], 0, 0, 0);
+#pragma unroll
+          for (int t = 0; t < T; ++t)
+            acc[t][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(xb[j][e], wb[t][j][e], acc[t][e & 1], 0, 0, 0);
         if (i + PD < nch) load(j, 16 * (i + PD));
       }
     }
   }
   // the waves' tiles through LDS, then one output per thread of the first 4 waves
 #pragma unroll
-  for (int v = 0; v < 4; ++v) red[wave][4 * q + v][c] = acc[0][v] + acc[1][v];
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) red[t][wave][4 * q + v][c] = acc[t][0][v] + acc[t][1][v];
   __syncthreads();
   if (tid < 256) {
     const int r = tid >> 4, col = tid & 15;
     const int m = m0 + r, n = n0 + col;
-    float s = 0.f;
+    float s[T];
 #pragma unroll
-    for (int w = 0; w < kLinWaves; ++w) s += red[w][r][col];
-    if (m < p.M && n < grp.n) p.y[(int64_t)m * p.ldy + grp.col_off + n] = s;
+    for (int t = 0; t < T; ++t) {
+      s[t] = 0.f;
+#pragma unroll
+      for (int w = 0; w < kLinWaves; ++w) s[t] += red[t][w][r][col];
+    }
+    if (m < p.M && n < grp.n) {
+      float* y = p.y + (int64_t)m * p.ldy + grp.col_off + n;
+      if constexpr (GATE) *y = s[0] * ops::sigmoid_fast(s[0]) * s[1];
+      else *y = s[0];
+    }
   }
 }
 

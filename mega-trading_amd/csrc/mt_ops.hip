@@ -530,9 +530,12 @@ int mt_apply_rope(const void* q, const void* k, void* q_out, void* k_out, int B,
   return e == hipSuccess ? ok() : fail((int)e, "launch failed: %s", hipGetErrorString(e));
 }
 
-int mt_linear_rows(const void* x, int64_t x_row_stride, const void* const* weights, const int* out_features,
-                   const int64_t* w_row_strides, int groups, void* y, int64_t y_row_stride, int rows, int in_features,
-                   int dtype, void* stream) {
+namespace {
+// The checks and launch of mt_linear_rows and, with gate, mt_linear_rows_gate
+// (two groups of equal width whose products never leave the workgroup).
+int linear_rows(const void* x, int64_t x_row_stride, const void* const* weights, const int* out_features,
+                const int64_t* w_row_strides, int groups, void* y, int64_t y_row_stride, int rows, int in_features,
+                int dtype, bool gate, void* stream) {
   if (dtype != MT_DTYPE_FP32 && dtype != MT_DTYPE_BF16 && dtype != MT_DTYPE_FP16)
     return fail(MT_E_DTYPE, "x dtype code %d unsupported", dtype);
   if (groups < 1 || groups > mt::kLinGroups)
@@ -572,6 +575,12 @@ int mt_linear_rows(const void* x, int64_t x_row_stride, const void* const* weigh
     cols += out_features[g];
     tiles += (out_features[g] + mt::kLinCols - 1) / mt::kLinCols;
   }
+  if (gate) {
+    if (out_features[0] != out_features[1])
+      return fail(MT_E_SHAPE, "gate and up must have one width (got %d and %d)", out_features[0], out_features[1]);
+    cols /= 2;
+    tiles /= 2;
+  }
   if (cols > 0x7fffffffLL) return fail(MT_E_SHAPE, "too many output columns (%lld)", (long long)cols);
   if (y_row_stride < cols) return fail(MT_E_STRIDE, "y row stride %lld must be >= %lld", (long long)y_row_stride,
                                        (long long)cols);
@@ -579,15 +588,36 @@ int mt_linear_rows(const void* x, int64_t x_row_stride, const void* const* weigh
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid((unsigned)(tiles * ((rows + 15) / 16))), block(64 * mt::kLinWaves);
   // every chunk of a lane in flight at once up to K = 1536 (12 chunks of 4 values per lane)
-#define MT_LINEAR(XT)                                                                                        \
-  if (in_features <= 128 * 12) hipLaunchKernelGGL((mt::linear_rows_f32_kernel<12, XT>), grid, block, 0, st, p); \
-  else hipLaunchKernelGGL((mt::linear_rows_f32_kernel<4, XT>), grid, block, 0, st, p)
+#define MT_LINEAR_G(XT, G)                                                                                      \
+  if (in_features <= 128 * 12) hipLaunchKernelGGL((mt::linear_rows_f32_kernel<12, XT, G>), grid, block, 0, st, p); \
+  else hipLaunchKernelGGL((mt::linear_rows_f32_kernel<4, XT, G>), grid, block, 0, st, p)
+#define MT_LINEAR(XT)                 \
+  if (gate) { MT_LINEAR_G(XT, true); } \
+  else { MT_LINEAR_G(XT, false); }
   if (dtype == MT_DTYPE_FP32) { MT_LINEAR(float); }
   else if (dtype == MT_DTYPE_BF16) { MT_LINEAR(mt::BF16); }
   else { MT_LINEAR(mt::FP16); }
 #undef MT_LINEAR
+#undef MT_LINEAR_G
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? ok() : fail((int)e, "launch failed: %s", hipGetErrorString(e));
+}
+}  // namespace
+
+int mt_linear_rows(const void* x, int64_t x_row_stride, const void* const* weights, const int* out_features,
+                   const int64_t* w_row_strides, int groups, void* y, int64_t y_row_stride, int rows, int in_features,
+                   int dtype, void* stream) {
+  return linear_rows(x, x_row_stride, weights, out_features, w_row_strides, groups, y, y_row_stride, rows, in_features,
+                     dtype, false, stream);
+}
+
+int mt_linear_rows_gate(const void* x, int64_t x_row_stride, const void* w_gate, const void* w_up,
+                        int64_t gate_row_stride, int64_t up_row_stride, void* y, int64_t y_row_stride, int rows,
+                        int in_features, int out_features, int dtype, void* stream) {
+  const void* const weights[2] = {w_gate, w_up};
+  const int outs[2] = {out_features, out_features};
+  const int64_t lds[2] = {gate_row_stride, up_row_stride};
+  return linear_rows(x, x_row_stride, weights, outs, lds, 2, y, y_row_stride, rows, in_features, dtype, true, stream);
 }
 
 int mt_topk_sample(const void* logits, int64_t row_stride, const void* noise, int64_t noise_row_stride, int rows,

@@ -57,6 +57,7 @@ from .ops import swiglu_gate_packed as _hip_swiglu_gate_packed
 from .ops import MAX_SAMPLE_VOCAB as _MAX_SAMPLE_VOCAB
 from .ops import topk_sample as _hip_topk_sample
 from .projection import project as _project
+from .projection import gate_rows as _gate_rows
 from .projection import project_packed as _project_packed
 
 __all__ = ["TradingModel", "LlamaDecoderBlock", "LlamaAttention", "SwiGLU", "RMSNorm", "RotaryEmbedding",
@@ -478,7 +479,9 @@ class SwiGLU(nn.Module):
     def forward(self, hidden: torch.Tensor) -> torch.Tensor:
         if self.operator_backend == "hip":
             # one GEMM for w1 and w3, the gate on its packed output, split-K dW
-            gated = _hip_swiglu_gate_packed(_project_packed(hidden, (self.w1.weight, self.w3.weight)))
+            gated = _gate_rows(hidden, self.w1.weight, self.w3.weight)  # a decode step's few rows
+            if gated is None:
+                gated = _hip_swiglu_gate_packed(_project_packed(hidden, (self.w1.weight, self.w3.weight)))
             return _project_packed(self.dropout(gated), (self.w2.weight,))
         gate = self.w1(hidden)
         up = self.w3(hidden)

@@ -31,14 +31,14 @@ Backward:
 from __future__ import annotations
 
 import ctypes
-from typing import Sequence
+from typing import Optional, Sequence
 
 import torch
 
 from . import _native
 from .gemm_tuning import tuned_gemms
 
-__all__ = ["project", "project_packed", "split_k_chunks"]
+__all__ = ["gate_rows", "project", "project_packed", "split_k_chunks"]
 
 _MIN_CHUNK_ROWS = 1024
 _MAX_CHUNKS = 16
@@ -156,6 +156,26 @@ def linear_rows(x: torch.Tensor, weights: list[torch.Tensor]) -> torch.Tensor:
     return y
 
 
+@torch.library.custom_op("mega_trading_amd::linear_rows_gate", mutates_args=(), device_types="cuda")
+def linear_rows_gate(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor) -> torch.Tensor:
+    """silu(x @ w_gate.T) * (x @ w_up.T) [rows, out], fp32, for x and the
+    weights as ``linear_rows`` takes them (``mt_linear_rows_gate``)."""
+    lib = _native.load()
+    rows, k = x.shape
+    y = torch.empty((rows, w_gate.shape[0]), device=x.device, dtype=torch.float32)
+    with torch.cuda.device(x.device):
+        rc = lib.mt_linear_rows_gate(x.data_ptr(), x.stride(0), w_gate.data_ptr(), w_up.data_ptr(), w_gate.stride(0),
+                                     w_up.stride(0), y.data_ptr(), y.stride(0), rows, k, w_gate.shape[0],
+                                     _X_DTYPES[x.dtype], torch.cuda.current_stream(x.device).cuda_stream)
+    _native.check(rc, "mt_linear_rows_gate")
+    return y
+
+
+@linear_rows_gate.register_fake
+def _linear_rows_gate_fake(x, w_gate, w_up):
+    return x.new_empty((x.shape[0], w_gate.shape[0]), dtype=torch.float32)
+
+
 @linear_rows.register_fake
 def _linear_rows_fake(x, weights):
     return x.new_empty((x.shape[0], sum(w.shape[0] for w in weights)))
@@ -180,6 +200,19 @@ def project_packed(x: torch.Tensor, weights: Sequence[torch.Tensor]) -> torch.Te
     if _rows_path(x2, weights, dtype):
         return linear_rows(x2, list(weights)).view(*x.shape[:-1], -1)
     return _Project.apply(x, dtype, *weights)
+
+
+def gate_rows(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor) -> Optional[torch.Tensor]:
+    """The SwiGLU's ``silu(x @ w_gate.T) * (x @ w_up.T)`` for the few rows of a
+    decode step, in one launch that keeps both products in the workgroup (the
+    values of ``swiglu_gate_packed`` on ``project_packed``'s output); None where
+    the few-row product does not apply."""
+    _check(x, (w_gate, w_up))
+    x2 = x.reshape(-1, x.shape[-1])
+    if (w_gate.shape != w_up.shape or w_gate.shape[0] % 8
+            or not _rows_path(x2, (w_gate, w_up), _compute_dtype(x, (w_gate, w_up)))):
+        return None
+    return linear_rows_gate(x2, w_gate, w_up).view(*x.shape[:-1], -1)
 
 
 def project(x: torch.Tensor, weights: Sequence[torch.Tensor]) -> tuple[torch.Tensor, ...]:

@@ -107,3 +107,19 @@ def test_linear_rows_in_a_recorded_graph_matches_eager():
     graph.replay()
     torch.cuda.synchronize()
     assert torch.equal(static, proj.linear_rows(x, ws))
+
+
+@pytest.mark.parametrize("rows,k,n,dt", [(1, 128, 8, torch.float32), (32, 512, 1408, torch.float32),
+                                         (17, 1664, 40, torch.float32), (64, 256, 24, torch.bfloat16)])
+def test_gate_rows_equals_the_two_launches(rows, k, n, dt):
+    ops = importlib.import_module("mega-trading_amd.ops")
+    g = torch.Generator().manual_seed(rows + n)
+    x = torch.randn(rows, 1, k, generator=g).to(dt).cuda()
+    ws = [(torch.randn(n, k, generator=g) * 2 / k ** 0.5).cuda() for _ in range(2)]
+    with torch.no_grad():
+        got = proj.gate_rows(x, *ws)
+        ref = ops.swiglu_gate_packed(proj.project_packed(x, ws))
+        assert proj.gate_rows(x.repeat(65, 1, 1), *ws) is None and proj.gate_rows(x, ws[0][:7], ws[1][:7]) is None
+    assert got.shape == (rows, 1, n)
+    # silu(g) u in one expression: its two roundings may fuse, 2 ulp of fp32
+    torch.testing.assert_close(got, ref, rtol=2.4e-7, atol=1e-12)
