@@ -13,18 +13,20 @@
 // A row lives on one CU, so the kernel is bound by its chain of dependent
 // steps, not by bandwidth; what it avoids is block-wide barriers.
 //
-// k <= 64: every wave finds the k-th largest of its 64 lane maxima (one ballot
-// and count per bit, no barrier); at least k keys of the row are >= the
-// largest of these 16 bounds, so the k-th key is too.  The keys at or above
-// the bound (about 200 of 16384 random ones at k = 16) go to LDS in index
-// order of (wave, slot, lane); a candidate is kept when fewer than k
-// candidates are larger, which keeps every tie at the k-th value, as the
-// reference's `logits < values[:, [-1]]` mask does.  One wave then takes the
+// k <= 1024: every wave finds the ceil(k / 16)-th and the k-th largest of its 64
+// lane maxima (one ballot and count per bit, no barrier).  At least k keys of the
+// row are >= the smallest of the 16 first bounds, and >= the largest of the
+// second ones, so the k-th key is too.  The keys at or above the larger of the two
+// (about 60 of 16384 random ones at k = 16, 110 at k = 50) go to LDS in index
+// order of (wave, slot, lane); a candidate is kept when fewer than k candidates
+// are larger, which keeps every tie at the k-th value, as the reference's
+// `logits < values[:, [-1]]` mask does.  One wave then takes the
 // maximum, the sum of exp(x - max), p = exp(x - max) / sum and the first
 // index of the largest p / E, reading E for the candidates alone: four
-// barriers in all.  32 rows of 16384, k = 16: 24.0 -> 12.4 us a launch.
+// barriers in all.  32 rows of 16384, k = 16: 24.0 -> 9.7 us a launch,
+// k = 50: 24.6 -> 12.5; 45 of 1385, k = 50: 18.7 -> 12.2.
 //
-// k > 64, or more than kSampleCand candidates (long runs of equal logits): the
+// k > 1024, or more than kSampleCand candidates (long runs of equal logits): the
 // k-th key bit by bit with block-wide counts (32 of them, two barriers each),
 // then block-wide reductions over the row (the 24.0 us).
 #pragma once
@@ -58,14 +60,14 @@ __device__ __forceinline__ float block_reduce(float v, float* buf) {
 
 constexpr int kSampleCand = 1024;   // candidates held in LDS
 constexpr int kSampleWaves = kSampleThreads / 64;
-constexpr int kSampleWaveK = 64;    // largest k of the candidate path: a wave's lane maxima hold a k-th
+constexpr int kSampleWaveK = 64 * kSampleWaves;  // largest k of the candidate path: the lane maxima hold a k-th
 
 __device__ __forceinline__ float sample_unkey(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? k & 0x7fffffffu : ~k);
 }
 
 struct SampleCand {
-  uint32_t bound[kSampleWaves];
+  uint32_t bound[2][kSampleWaves];
   int count[kSampleWaves];
   uint32_t key[kSampleCand];
   int idx[kSampleCand];  // vocabulary index; -1 once dropped
@@ -81,16 +83,25 @@ __device__ __forceinline__ bool sample_candidates(const uint32_t (&key)[EPT], co
   uint32_t mx = 0u;
 #pragma unroll
   for (int j = 0; j < EPT; ++j) mx = max(mx, key[j]);
-  // the k-th largest lane maximum (0 while the wave holds fewer than k values)
-  uint32_t t = 0u;
+  // the k1-th and k-th largest lane maxima (0 where the wave holds fewer values)
+  const int k1 = (k + kSampleWaves - 1) / kSampleWaves;
+  uint32_t t1 = 0u, t2 = 0u;
   for (int bit = 31; bit >= 0; --bit) {
-    const uint32_t cand = t | (1u << bit);
-    if (__popcll(__ballot(mx >= cand)) >= k) t = cand;
+    const uint32_t c1 = t1 | (1u << bit), c2 = t2 | (1u << bit);
+    if (__popcll(__ballot(mx >= c1)) >= k1) t1 = c1;
+    if (__popcll(__ballot(mx >= c2)) >= k) t2 = c2;
   }
-  if (lane == 0) s.bound[wave] = t;
+  if (lane == 0) {
+    s.bound[0][wave] = t1;
+    s.bound[1][wave] = t2;
+  }
   __syncthreads();
 #pragma unroll
-  for (int w = 0; w < kSampleWaves; ++w) t = max(t, s.bound[w]);
+  for (int w = 0; w < kSampleWaves; ++w) {
+    t1 = min(t1, s.bound[0][w]);
+    t2 = max(t2, s.bound[1][w]);
+  }
+  const uint32_t t = max(t1, t2);
   int mine = 0;
 #pragma unroll
   for (int j = 0; j < EPT; ++j) mine += __popcll(__ballot(key[j] >= t && tid + j * kSampleThreads < V));

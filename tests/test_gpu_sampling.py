@@ -56,8 +56,11 @@ def test_topk_sample_keeps_every_tie_at_the_kth_value():
 
 
 @pytest.mark.parametrize("rows,vocab,k,kind", [
-    (4, 4096, 64, "normal"),      # the largest k of the candidate path
-    (4, 4096, 65, "normal"),      # the first k counted block-wide
+    (4, 4096, 64, "normal"),      # the largest k a wave's lane maxima bound by themselves
+    (4, 4096, 65, "normal"),
+    (4, 32768, 50, "normal"),
+    (2, 2000, 1024, "normal"),    # the largest k of the candidate path
+    (2, 2000, 1025, "normal"),    # the first k counted block-wide
     (3, 8192, 16, "ties"),        # more ties than the candidate list holds
     (3, 1024, 3, "equal"),        # every logit a candidate, exactly the list's size
     (3, 1025, 3, "equal"),        # one more than it holds
