@@ -6,10 +6,20 @@
 // fallback (:88-111).  These kernels compute both in full fp32: the MFMA
 // multiplies fp32 operands exactly and accumulates in fp32, P and dS stay fp32
 // (the reference casts P to V's dtype, fp32 here, :340), and the softmax runs
-// in fp32.  They favour simplicity over speed: one wave owns 32 query rows (or
-// 32 keys), reads its K / V (or Q / dO) rows straight from global memory (no
-// LDS staging, no sharing across the group's heads beyond the L2) and runs the
-// diagonal tile masked.
+// in fp32.
+//
+// What bounds them is the fp32 MFMA (64 cycles for 32 x 32 x 2 products; a
+// library product sustains 154 TFLOP/s).  One wave owns 32 query rows (or 32
+// keys) and works on 32 x 32 score tiles; the tiles it multiplies come into its
+// own LDS block by asynchronous copies of whole rows, each issued as soon as the
+// tile before it has been read for the last time and waited for (by count)
+// only where its first operand is read, so a wave needs no barrier and the
+// copies run behind the MFMAs of the phases between.  Read straight from global
+// memory, a row per lane with 16 bytes from each of 64 cache lines a load, the
+// same tiles left the MFMAs idle two thirds of the time.  Measured, forward +
+// backward with RoPE: 8 x 512, 16 / 4 heads of 64: 362 -> 238 us; 4 x 1000, 8 / 2
+// of 64: 441 -> 284; 2 x 1024, 16 / 4 of 128: 1086 -> 660; 2 x 256, 4 / 2 of 32:
+// 48.6 -> 33.0.
 //
 // MFMA layout (32x32x2, fp32): A[m][k] comes from lane m + 32 k, B[k][n] from
 // lane n + 32 k, and lane l holds C[m][n = l % 32] for m = 8 (i / 4) + 4 (l / 32)
@@ -74,26 +84,131 @@ __global__ __launch_bounds__(256) void rope_f32_kernel(const float* x, int64_t s
 }
 
 // ---------------------------------------------------------------------------
-// Forward: online softmax over 32-key tiles, O and LSE.
+// LDS tiles of fp32 rows: a row of D floats is laid out, swizzled and copied as
+// a row of 2 D 16-bit values (lds_tile.h).
 // ---------------------------------------------------------------------------
-template <int D, bool ROPE>
-__global__ __launch_bounds__(256) void attn_fwd_f32_kernel(AttnParams p) {
+// Copies of 32 rows by one wave (lds wave-uniform): the offsets of 16 rows, the swizzle's period,
+// are kept and the scalar base moves for the other 16.
+template <int D>
+struct F32Stager {
+  using TL = Tile<2 * D>;
+  static constexpr int N = TL::NC / 4;      // 1 KB copies of 16 rows
+  static constexpr int COPIES = 2 * N;      // of a tile, whatever path it takes
+  uint32_t voff[N];
+  int lane_;
+
+  static __device__ __forceinline__ void place(int i, int lane, int& row, int& chunk) {
+    const int f = i * 64 + lane;
+    row = f / TL::NC;
+    chunk = (f % TL::NC) ^ TL::swz(row);
+  }
+  __device__ __forceinline__ void init(int64_t row_stride, int lane) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      int row, chunk;
+      place(i, lane, row, chunk);
+      voff[i] = (uint32_t)(row * (int)row_stride + chunk * 4) * 4u;
+    }
+    lane_ = lane;
+  }
+  // rows [row0, row0 + 32) of the matrix at src; rows past T - 1 copy row T - 1
+  __device__ __forceinline__ void stage(char* lds, const float* src, int64_t row_stride, int row0, int T) const {
+    if (row0 + 32 <= T) {
+      const uint32_t l0 = lds_addr(lds);
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+          lds_dma16_s(src + (int64_t)(row0 + 16 * g) * row_stride, voff[i], l0 + (g * N + i) * 1024);
+    } else {
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          int row, chunk;
+          place(i, lane_, row, chunk);
+          const int grow = min(row0 + 16 * g + row, T - 1);
+          lds_dma16(reinterpret_cast<const uint16_t*>(src + (int64_t)grow * row_stride + chunk * 4),
+                    lds + (g * N + i) * 1024);
+        }
+    }
+  }
+};
+
+// Operand reads of such a tile.
+//  * row: lane (row l32, half hh) reads d values hh D/2 + 4 j .. + 3 (the score
+//    contraction's pairing); 16 consecutive rows of a chunk column cover 256
+//    distinct bytes.
+//  * tr: lane reads d = 32 dt + l32 of the row its accumulator slot j refers to.
+template <int D>
+struct F32Tile {
+  using TL = Tile<2 * D>;
+  int rbase, tbase;
+  __device__ __forceinline__ F32Tile(int l32, int hh)
+      : rbase(l32 * TL::RB + (((hh * (D / 8)) ^ TL::swz(l32)) << 4)),
+        tbase(4 * hh * TL::RB + (((l32 >> 2) ^ hh) << 4) + (l32 & 3) * 4) {}
+  __device__ __forceinline__ f32x4 row(const char* lds, int j) const {
+    return *reinterpret_cast<const f32x4*>(lds + (rbase ^ (j << 4)));
+  }
+  // the swizzle of row 8 (j / 4) + 4 hh + j % 4 without hh, which tbase holds
+  static constexpr int tr_swz(int j) {
+    return TL::NC == 8 ? (((j >> 1) & 1) << 2) | (((j >> 2) & 1) << 1) : ((j & 3) << 2) | (((j >> 2) & 1) << 1);
+  }
+  __device__ __forceinline__ float tr(const char* lds, int j, int dt) const {
+    return *reinterpret_cast<const float*>(lds + (8 * (j >> 2) + (j & 3)) * TL::RB +
+                                           (tbase ^ (((8 * dt) ^ tr_swz(j)) << 4)));
+  }
+};
+
+// All but the wave's newest N copies are done; no LDS read moves across.
+template <int N>
+__device__ __forceinline__ void f32_copies_done() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// every LDS read a wave has issued is done, before a copy overwrites what they read
+__device__ __forceinline__ void f32_reads_done() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
+
+// ---------------------------------------------------------------------------
+// Forward: online softmax over 32-key tiles, O and LSE.  SPLIT = 4: the tiles of
+// a row block are dealt to the 4 waves of a workgroup, whose (O, m, l) are
+// merged; SPLIT = 1: every wave has a row block of its own.
+// ---------------------------------------------------------------------------
+template <int D, bool ROPE, int SPLIT>
+__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_fwd_f32_kernel(AttnParams p) {
   constexpr int HD = D / 2;  // d values per lane
   constexpr int DT = D / 32;
-  __shared__ f32x4 red_o[3][DT * 4][64];  // waves 1-3: [wave - 1][dt, g][lane] unnormalised O
-  __shared__ f32x2 red_ml[3][64];         // and (m, l)
+  using TL = Tile<2 * D>;
+  constexpr int BUF = 2 * 32 * TL::RB;  // a wave's K and V tiles
+  __shared__ __attribute__((aligned(1024))) char smem[4 * BUF];
+  // after the loop, waves 1-3: unnormalised O [wave - 1][dt, g][lane] and (m, l)
+  f32x4 (*red_o)[DT * 4][64] = reinterpret_cast<f32x4 (*)[DT * 4][64]>(smem);
+  __shared__ f32x2 red_ml[3][64];
   const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nblk = (p.T + 31) / 32;
-  const int t = blockIdx.x;
-  if (t >= p.B * p.Hq * nblk) return;  // (workgroup-uniform)
+  const int t = SPLIT == 4 ? (int)blockIdx.x : fold_order(blockIdx.x, gridDim.x, p.fwd_fold) * 4 + wave;
+  if (t >= p.B * p.Hq * nblk) return;  // (workgroup-uniform with SPLIT = 4; no barriers otherwise)
   const F32Task task = f32_task(t, p.B, p.Hq, nblk, true);
   const int kvh = task.h / p.R;
   const int row = task.blk * 32 + l32;
   const int rc = min(row, p.T - 1);
+  const int kt0 = SPLIT == 4 ? wave : 0;
+  const float* kbase = fptr(p.k) + task.b * p.sk[0] + (int64_t)kvh * p.sk[1];
+  const float* vbase = fptr(p.v) + task.b * p.sv[0] + (int64_t)kvh * p.sv[1];
+  F32Stager<D> kst, vst;
+  kst.init(p.sk[2], lane);
+  vst.init(p.sv[2], lane);
+  char* K = smem + wave * BUF;
+  char* V = K + 32 * TL::RB;
+  if (kt0 <= task.blk) {
+    kst.stage(K, kbase, p.sk[2], kt0 * 32, p.T);
+    vst.stage(V, vbase, p.sv[2], kt0 * 32, p.T);
+  }
 
   // the lane's half of its query row, rotated if RoPE (and written to q_rot,
-  // by wave 0)
+  // by wave 0 of a split block)
   float qv[HD];
   {
     const float* qr = fptr(p.q) + task.b * p.sq[0] + (int64_t)task.h * p.sq[1] + (int64_t)rc * p.sq[2] + hh * HD;
@@ -106,42 +221,48 @@ __global__ __launch_bounds__(256) void attn_fwd_f32_kernel(AttnParams p) {
         const f32x2 sn = *reinterpret_cast<const f32x2*>(p.sin + (int64_t)rc * (D / 2) + d0 / 2);
         x = f32x4{x[0] * cs[0] - x[1] * sn[0], x[0] * sn[0] + x[1] * cs[0], x[2] * cs[1] - x[3] * sn[1],
                   x[2] * sn[1] + x[3] * cs[1]};
-        if (wave == 0 && row < p.T)
+        if ((SPLIT == 1 || wave == 0) && row < p.T)
           *reinterpret_cast<f32x4*>(fptr(p.qrot) + (((int64_t)task.b * p.Hq + task.h) * p.T + row) * D + d0) = x;
       }
 #pragma unroll
       for (int c = 0; c < 4; ++c) qv[4 * j + c] = x[c];
     }
   }
-  const float* kbase = fptr(p.k) + task.b * p.sk[0] + (int64_t)kvh * p.sk[1];
-  const float* vbase = fptr(p.v) + task.b * p.sv[0] + (int64_t)kvh * p.sv[1];
   const float c2 = p.scale_log2;
+  const F32Tile<D> tile(l32, hh);
 
   f32x16 oacc[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) zero16(oacc[dt]);
   float m = -INFINITY, l = 0.f;
-  // the key tiles on or left of the diagonal are dealt to the 4 waves in turn;
-  // each keeps its own running offset and sums, merged below
-  for (int kt = wave; kt <= task.blk; kt += 4) {
+  for (int kt = kt0; kt <= task.blk; kt += SPLIT) {
+    const bool more = kt + SPLIT <= task.blk;
+    // K is here; V may still be on its way (the first time the wave also has its
+    // Q loads and Q_rot stores behind the copies)
+    if (kt == kt0) f32_copies_done<0>();
+    else f32_copies_done<F32Stager<D>::COPIES>();
     // S^T (lane = query, slots = keys)
-    const float* kr = kbase + (int64_t)min(kt * 32 + l32, p.T - 1) * p.sk[2] + hh * HD;
     f32x16 s = {};
 #pragma unroll
     for (int j = 0; j < HD / 4; ++j) {
-      const f32x4 k4 = *reinterpret_cast<const f32x4*>(kr + 4 * j);
+      const f32x4 k4 = tile.row(K, j);
 #pragma unroll
       for (int c = 0; c < 4; ++c) s = mfma_f32(k4[c], qv[4 * j + c], s);
     }
+    f32_reads_done();
+    if (more) kst.stage(K, kbase, p.sk[2], (kt + SPLIT) * 32, p.T);
+    if (kt == task.blk) {  // the diagonal; tiles left of it have every key <= every row
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (f32_slot_row(i, hh) > l32) s[i] = -INFINITY;
+    }
+    // the diagonal tile holds key 32 kt <= row, so m is finite after a wave's first tile
     float mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int key = kt * 32 + f32_slot_row(i, hh);
-      s[i] = (key <= row && key < p.T) ? s[i] * c2 : -INFINITY;
+      s[i] *= c2;
       mx = fmaxf(mx, s[i]);
     }
-    // every tile left of the diagonal is unmasked and the diagonal tile holds
-    // key 32 kt <= row, so m is finite after a wave's first tile
     const float mnew = fmaxf(m, max_with_partner(mx));
     const float alpha = exp2_fast(m - mnew);
     float ps = 0.f;
@@ -157,13 +278,17 @@ __global__ __launch_bounds__(256) void attn_fwd_f32_kernel(AttnParams p) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) oacc[dt][i] *= alpha;
     // O^T += V^T P^T over the tile's 32 keys
+    if (more) f32_copies_done<F32Stager<D>::COPIES>();
+    else f32_copies_done<0>();
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const float* vr = vbase + (int64_t)min(kt * 32 + f32_slot_row(j, hh), p.T - 1) * p.sv[2] + l32;
+    for (int j = 0; j < 16; ++j)
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) oacc[dt] = mfma_f32(vr[32 * dt], s[j], oacc[dt]);
-    }
+      for (int dt = 0; dt < DT; ++dt) oacc[dt] = mfma_f32(tile.tr(V, j, dt), s[j], oacc[dt]);
+    f32_reads_done();
+    if (more) vst.stage(V, vbase, p.sv[2], (kt + SPLIT) * 32, p.T);
   }
+  if constexpr (SPLIT == 4) {
+  __syncthreads();  // every wave's tiles are read: the block is reused for the merge
   // merge the four waves' (O, m, l) with the log-sum-exp rule (a wave that
   // had no tile has m = -inf and contributes nothing); m is the same on a
   // lane and its lane^32 partner
@@ -207,6 +332,7 @@ __global__ __launch_bounds__(256) void attn_fwd_f32_kernel(AttnParams p) {
     }
     m = mm;
   }
+  }
   if (row >= p.T) return;
   const float lt = sum_with_partner(l);
   const float inv = 1.f / lt;
@@ -249,27 +375,43 @@ __global__ __launch_bounds__(256) void attn_bwd_prep_f32_kernel(AttnParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Backward dQ: per workgroup 32 query rows of one head; the 32-key tiles on
+// Backward dQ: per workgroup 32 query rows of one head (SPLIT = 4; SPLIT = 1 as
+// in the forward, the tiles of a row block on one wave); the 32-key tiles on
 // or left of the diagonal are dealt to the 4 waves in turn (each recomputes
 // S^T and dP^T for its tiles, lane = query: P = 2^(S c - LSE2), dS = P (dP -
 // delta), dQ^T += K^T dS^T), and the four partial sums are added through LDS.
 // ---------------------------------------------------------------------------
-template <int D, bool ROPE>
-__global__ __launch_bounds__(256) void attn_bwd_dq_f32_kernel(AttnParams p) {
+template <int D, bool ROPE, int SPLIT>
+__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_bwd_dq_f32_kernel(AttnParams p) {
   constexpr int HD = D / 2;
   constexpr int DT = D / 32;
-  __shared__ f32x4 red[3][DT * 4][64];  // waves 1-3: [wave - 1][dt, g][lane]
+  using TL = Tile<2 * D>;
+  constexpr int BUF = 2 * 32 * TL::RB;  // a wave's K and V tiles
+  __shared__ __attribute__((aligned(1024))) char smem[4 * BUF];
+  f32x4 (*red)[DT * 4][64] = reinterpret_cast<f32x4 (*)[DT * 4][64]>(smem);  // after the loop: waves 1-3
   const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nblk = (p.T + 31) / 32;
-  const int t = blockIdx.x;
-  if (t >= p.B * p.Hq * nblk) return;  // (workgroup-uniform)
+  const int t = SPLIT == 4 ? (int)blockIdx.x : fold_order(blockIdx.x, gridDim.x, p.fwd_fold) * 4 + wave;
+  if (t >= p.B * p.Hq * nblk) return;  // (workgroup-uniform with SPLIT = 4; no barriers otherwise)
   const F32Task task = f32_task(t, p.B, p.Hq, nblk, true);
   const int kvh = task.h / p.R;
   const int row = task.blk * 32 + l32;
   const int rc = min(row, p.T - 1);
   const int64_t rowbase = ((int64_t)task.b * p.Hq + task.h) * p.T;
 
+  const int kt0 = SPLIT == 4 ? wave : 0;
+  const float* kbase = fptr(p.k) + task.b * p.sk[0] + (int64_t)kvh * p.sk[1];
+  const float* vbase = fptr(p.v) + task.b * p.sv[0] + (int64_t)kvh * p.sv[1];
+  F32Stager<D> kst, vst;
+  kst.init(p.sk[2], lane);
+  vst.init(p.sv[2], lane);
+  char* K = smem + wave * BUF;
+  char* V = K + 32 * TL::RB;
+  if (kt0 <= task.blk) {
+    vst.stage(V, vbase, p.sv[2], kt0 * 32, p.T);
+    kst.stage(K, kbase, p.sk[2], kt0 * 32, p.T);
+  }
   float qv[HD], gv[HD];
   {
     const float* qr = fptr(p.q) + task.b * p.sq[0] + (int64_t)task.h * p.sq[1] + (int64_t)rc * p.sq[2] + hh * HD;
@@ -287,41 +429,55 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_f32_kernel(AttnParams p) {
   }
   const float nl2 = p.nlse2[rowbase + rc];
   const float nd = p.ndelta[rowbase + rc];
-  const float* kbase = fptr(p.k) + task.b * p.sk[0] + (int64_t)kvh * p.sk[1];
-  const float* vbase = fptr(p.v) + task.b * p.sv[0] + (int64_t)kvh * p.sv[1];
   const float c2 = p.scale_log2;
+  const F32Tile<D> tile(l32, hh);
 
   f32x16 dq[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) zero16(dq[dt]);
-  for (int kt = wave; kt <= task.blk; kt += 4) {
-    const int kc = min(kt * 32 + l32, p.T - 1);
-    const float* kr = kbase + (int64_t)kc * p.sk[2] + hh * HD;
-    const float* vr = vbase + (int64_t)kc * p.sv[2] + hh * HD;
+  // dP first, then S: V's next tile is copied behind S and dQ, K's behind the next dP
+  for (int kt = kt0; kt <= task.blk; kt += SPLIT) {
+    const bool more = kt + SPLIT <= task.blk;
+    if (kt == kt0) f32_copies_done<0>();
+    else f32_copies_done<F32Stager<D>::COPIES>();
     f32x16 s = {}, dp = {};
 #pragma unroll
     for (int j = 0; j < HD / 4; ++j) {
-      const f32x4 k4 = *reinterpret_cast<const f32x4*>(kr + 4 * j);
-      const f32x4 v4 = *reinterpret_cast<const f32x4*>(vr + 4 * j);
+      const f32x4 v4 = tile.row(V, j);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        s = mfma_f32(k4[c], qv[4 * j + c], s);
-        dp = mfma_f32(v4[c], gv[4 * j + c], dp);
-      }
+      for (int c = 0; c < 4; ++c) dp = mfma_f32(v4[c], gv[4 * j + c], dp);
+    }
+    f32_reads_done();
+    if (more) {
+      vst.stage(V, vbase, p.sv[2], (kt + SPLIT) * 32, p.T);
+      f32_copies_done<F32Stager<D>::COPIES>();
+    } else {
+      f32_copies_done<0>();
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int key = kt * 32 + f32_slot_row(i, hh);
-      const float pv = (key <= row && key < p.T && row < p.T) ? exp2_fast(__builtin_fmaf(s[i], c2, nl2)) : 0.f;
-      s[i] = pv * (dp[i] + nd);  // dS
+    for (int j = 0; j < HD / 4; ++j) {
+      const f32x4 k4 = tile.row(K, j);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) s = mfma_f32(k4[c], qv[4 * j + c], s);
     }
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const float* kj = kbase + (int64_t)min(kt * 32 + f32_slot_row(j, hh), p.T - 1) * p.sk[2] + l32;
+    for (int i = 0; i < 16; ++i) s[i] = exp2_fast(__builtin_fmaf(s[i], c2, nl2));
+    if (kt == task.blk) {
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) dq[dt] = mfma_f32(kj[32 * dt], s[j], dq[dt]);
+      for (int i = 0; i < 16; ++i)
+        if (f32_slot_row(i, hh) > l32) s[i] = 0.f;
     }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] *= dp[i] + nd;  // dS
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) dq[dt] = mfma_f32(tile.tr(K, j, dt), s[j], dq[dt]);
+    f32_reads_done();
+    if (more) kst.stage(K, kbase, p.sk[2], (kt + SPLIT) * 32, p.T);
   }
+  if constexpr (SPLIT == 4) {
+  __syncthreads();  // every wave's tiles are read: the block is reused for the sums
   // the four waves' partial sums: waves 1-3 hand theirs to wave 0
   if (wave > 0) {
 #pragma unroll
@@ -342,6 +498,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_f32_kernel(AttnParams p) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) dq[dt][4 * g + e] += a[e];
       }
+  }
   if (row >= p.T) return;
   float* out = fptr(p.out) + task.b * p.sout[0] + (int64_t)task.h * p.sout[1] + (int64_t)row * p.sout[2];
 #pragma unroll
@@ -367,12 +524,16 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_f32_kernel(AttnParams p) {
 // SIMDs, the longest walking every row of its heads).
 // ---------------------------------------------------------------------------
 template <int D, bool ROPE>
-__global__ __launch_bounds__(256) void attn_bwd_dkv_f32_kernel(AttnParams p) {
+__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_bwd_dkv_f32_kernel(AttnParams p) {
   constexpr int HD = D / 2;
   constexpr int DT = D / 32;
-  __shared__ f32x4 red[3][2 * DT * 4][64];  // waves 1-3: [wave - 1][dK / dV, dt, g][lane]
+  using TL = Tile<2 * D>;
+  constexpr int BUF = 2 * 32 * TL::RB + 256;  // a wave's Q rows, dO rows, and their -LSE log2(e) | -delta
+  constexpr int RED = 3 * 2 * DT * 4 * 64 * 16;
+  __shared__ __attribute__((aligned(1024))) char smem[4 * BUF > RED ? 4 * BUF : RED];
+  f32x4 (*red)[2 * DT * 4][64] = reinterpret_cast<f32x4 (*)[2 * DT * 4][64]>(smem);  // after the loop: waves 1-3
   const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nblk = (p.T + 31) / 32;
   const int t = blockIdx.x;
   if (t >= p.B * p.Hkv * nblk) return;  // (workgroup-uniform)
@@ -403,51 +564,98 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_f32_kernel(AttnParams p) {
     zero16(dv[dt]);
   }
   const int ntile = nblk - task.blk;  // row tiles per head on or below the diagonal
-  for (int u = wave; u < p.R * ntile; u += 4) {
-    const int r = u % p.R;
+  const int npair = p.R * ntile;
+  // Each wave copies the rows of its next pair into its own LDS block: Q behind
+  // dV, dO behind the next S.
+  char* Qt = smem + wave * BUF;
+  char* Gt = Qt + 32 * TL::RB;
+  const float* vec = reinterpret_cast<const float*>(Gt + 32 * TL::RB);
+  F32Stager<D> qst, gst;
+  qst.init(p.sq[2], lane);
+  gst.init(p.sdo[2], lane);
+  const F32Tile<D> tile(l32, hh);
+  auto stage_q = [&](int u) {
+    const int head = task.h * p.R + u % p.R, qt = task.blk + u / p.R;
+    qst.stage(Qt, fptr(p.q) + task.b * p.sq[0] + (int64_t)head * p.sq[1], p.sq[2], qt * 32, p.T);
+  };
+  auto stage_g = [&](int u) {
+    const int head = task.h * p.R + u % p.R, qt = task.blk + u / p.R;
+    gst.stage(Gt, fptr(p.dout) + task.b * p.sdo[0] + (int64_t)head * p.sdo[1], p.sdo[2], qt * 32, p.T);
+    // lanes 0-31: the rows' -LSE log2(e), lanes 32-63: -delta
+    lds_dma4((hh ? p.ndelta : p.nlse2) + ((int64_t)task.b * p.Hq + head) * p.T + min(qt * 32 + l32, p.T - 1),
+             Gt + 32 * TL::RB);
+  };
+  if (wave < npair) {
+    stage_q(wave);
+    stage_g(wave);
+  }
+  for (int u = wave; u < npair; u += 4) {
     const int qt = task.blk + u / p.R;
-    const int head = task.h * p.R + r;
-    const float* qbase = fptr(p.q) + task.b * p.sq[0] + (int64_t)head * p.sq[1];
-    const float* gbase = fptr(p.dout) + task.b * p.sdo[0] + (int64_t)head * p.sdo[1];
-    const int64_t rowbase = ((int64_t)task.b * p.Hq + head) * p.T;
-    {
-      // S and dP: rows m = the tile's queries, lane = key
-      const int qa = min(qt * 32 + l32, p.T - 1);
-      const float* qr = qbase + (int64_t)qa * p.sq[2] + hh * HD;
-      const float* gr = gbase + (int64_t)qa * p.sdo[2] + hh * HD;
-      f32x16 s = {}, dp = {};
+    const bool more = u + 4 < npair;
+    // S and dP: rows m = the tile's queries, lane = key
+    f32x16 s = {}, dp = {};
+    f32_copies_done<F32Stager<D>::COPIES + 1>();  // Q (dO and its vectors may still be on their way)
 #pragma unroll
-      for (int j = 0; j < HD / 4; ++j) {
-        const f32x4 q4 = *reinterpret_cast<const f32x4*>(qr + 4 * j);
-        const f32x4 g4 = *reinterpret_cast<const f32x4*>(gr + 4 * j);
+    for (int j = 0; j < HD / 4; ++j) {
+      const f32x4 q4 = tile.row(Qt, j);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          s = mfma_f32(q4[c], kv[4 * j + c], s);
-          dp = mfma_f32(g4[c], vv[4 * j + c], dp);
-        }
+      for (int c = 0; c < 4; ++c) s = mfma_f32(q4[c], kv[4 * j + c], s);
+      if constexpr (D > 64) {
+        if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // a few operands in flight, not all
       }
+    }
+    f32_copies_done<0>();
+#pragma unroll
+    for (int j = 0; j < HD / 4; ++j) {
+      const f32x4 g4 = tile.row(Gt, j);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) dp = mfma_f32(g4[c], vv[4 * j + c], dp);
+      if constexpr (D > 64) {
+        if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const f32x4 nl = *reinterpret_cast<const f32x4*>(vec + 8 * a + 4 * hh);
+      const f32x4 nd = *reinterpret_cast<const f32x4*>(vec + 32 + 8 * a + 4 * hh);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int i = 4 * a + c;
+        s[i] = exp2_fast(__builtin_fmaf(s[i], c2, nl[c]));
+        dp[i] += nd[c];
+      }
+    }
+    if (qt == task.blk || qt * 32 + 32 > p.T) {  // the diagonal, or rows past T
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int qrow = qt * 32 + f32_slot_row(i, hh);
-        const int qcl = min(qrow, p.T - 1);
-        const bool ok = key <= qrow && qrow < p.T && key < p.T;
-        const float pv = ok ? exp2_fast(__builtin_fmaf(s[i], c2, p.nlse2[rowbase + qcl])) : 0.f;
-        s[i] = pv;
-        dp[i] = pv * (dp[i] + p.ndelta[rowbase + qcl]);  // dS
-      }
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int qj = min(qt * 32 + f32_slot_row(j, hh), p.T - 1);
-        const float* qrj = qbase + (int64_t)qj * p.sq[2] + l32;
-        const float* grj = gbase + (int64_t)qj * p.sdo[2] + l32;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          dv[dt] = mfma_f32(grj[32 * dt], s[j], dv[dt]);
-          dk[dt] = mfma_f32(qrj[32 * dt], dp[j], dk[dt]);
-        }
+        if (key > qrow || qrow >= p.T) s[i] = 0.f;
       }
     }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) dp[i] *= s[i];  // dS
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) dk[dt] = mfma_f32(tile.tr(Qt, j, dt), dp[j], dk[dt]);
+      if constexpr (D > 64) {
+        if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    f32_reads_done();
+    if (more) stage_q(u + 4);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) dv[dt] = mfma_f32(tile.tr(Gt, j, dt), s[j], dv[dt]);
+      if constexpr (D > 64) {
+        if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    f32_reads_done();
+    if (more) stage_g(u + 4);
   }
+  __syncthreads();  // every wave's tiles are read: the block is reused for the sums
   // the four waves' partial sums: waves 1-3 hand theirs to wave 0
   if (wave > 0) {
 #pragma unroll
@@ -461,7 +669,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_f32_kernel(AttnParams p) {
   }
   __syncthreads();
   if (wave > 0) return;
-#pragma unroll
+#pragma unroll 1
   for (int w = 0; w < 3; ++w)
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)

@@ -59,7 +59,7 @@ struct Tile {
   // slot permutation of row r (period 16)
   static __device__ __forceinline__ int swz(int row) {
     if constexpr (NC == 8) return (((row >> 1) & 1) << 2) | ((row >> 2) & 3);
-    else if constexpr (NC == 16) return ((row & 3) << 2) | ((row >> 2) & 3);
+    else if constexpr (NC >= 16) return ((row & 3) << 2) | ((row >> 2) & 3);
     else return (row >> 2) & 3;  // NC == 4: four rows per 256 bytes
   }
 

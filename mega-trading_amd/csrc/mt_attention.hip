@@ -396,6 +396,22 @@ hipError_t launch_bwd(mt::AttnParams p, hipStream_t st, int stage) {
 
 // fp32 tensors: the fp32-MFMA kernels of attn_f32_kernels.h (K rotated by its
 // own pass with RoPE, as for 16-bit; no dK/dV head split)
+// Forward / dQ workgroups when every wave takes a row block of its own, else 0
+// (the tiles of a row block dealt to the 4 waves of a workgroup, merged in LDS).
+// Without the split no merge and no repeated Q load is paid, but the longest row
+// block bounds the launch, so the longer the rows the more row blocks it needs.
+// D = 64, forward + backward, split / whole, us: T = 64, 640 row blocks 66 / 53;
+// T = 89, 168 blocks 41 / 53; T = 200, 896 blocks 104 / 98; T = 384, 1152 blocks
+// 163 / 169; T = 512, 1024 blocks 170 / 191, 2048 blocks 265 / 238.
+int64_t f32_whole_blocks(mt::AttnParams& p) {
+  const int nblk = (p.T + 31) / 32;
+  const int64_t rows = (int64_t)p.B * p.Hq * nblk, blocks = (rows + 3) / 4;
+  const int cus = device_cus();
+  if (2 * rows < cus * (nblk <= 3 ? 4 : nblk <= 8 ? 7 : 10)) return 0;
+  p.fwd_fold = blocks > cus && blocks <= 2 * cus ? cus : 0;  // one resident round: heavy and light on each CU
+  return blocks;
+}
+
 template <int D, bool ROPE>
 hipError_t launch_fwd_f32(mt::AttnParams p, hipStream_t st, int) {
   if (ROPE) {
@@ -410,8 +426,10 @@ hipError_t launch_fwd_f32(mt::AttnParams p, hipStream_t st, int) {
     p.sk[1] = (int64_t)p.T * D;
     p.sk[2] = D;
   }
+  if (const int64_t whole = f32_whole_blocks(p))
+    return launch_main(mt::attn_fwd_f32_kernel<D, ROPE, 1>, dim3((unsigned)whole), dim3(256), st, p);
   const int64_t blocks = (int64_t)p.B * p.Hq * ((p.T + 31) / 32);  // one 4-wave workgroup per (batch, head, 32 rows)
-  return launch_main(mt::attn_fwd_f32_kernel<D, ROPE>, dim3((unsigned)blocks), dim3(256), st, p);
+  return launch_main(mt::attn_fwd_f32_kernel<D, ROPE, 4>, dim3((unsigned)blocks), dim3(256), st, p);
 }
 
 template <int D, bool ROPE>
@@ -424,8 +442,12 @@ hipError_t launch_bwd_f32(mt::AttnParams p, hipStream_t st, int stage) {
                        dim3(256), 0, st, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const int64_t blocks = (int64_t)p.B * p.Hq * nblk;  // one 4-wave workgroup per (batch, head, 32 rows)
-    e = launch_main(mt::attn_bwd_dq_f32_kernel<D, ROPE>, dim3((unsigned)blocks), dim3(256), st, p);
+    if (const int64_t whole = f32_whole_blocks(p)) {
+      e = launch_main(mt::attn_bwd_dq_f32_kernel<D, ROPE, 1>, dim3((unsigned)whole), dim3(256), st, p);
+    } else {
+      const int64_t blocks = (int64_t)p.B * p.Hq * nblk;  // one 4-wave workgroup per (batch, head, 32 rows)
+      e = launch_main(mt::attn_bwd_dq_f32_kernel<D, ROPE, 4>, dim3((unsigned)blocks), dim3(256), st, p);
+    }
     if (e != hipSuccess) return e;
   }
   if (stage & 2) {

@@ -113,3 +113,22 @@ def test_the_checks_catch_the_hazards():
     assert _writes("s_mov_b64 s[10:11], s[20:21]", {"s10", "s11"})
     assert not _writes("global_load_lds_dword v185, s[10:11]", {"s10", "s11"})
     assert _wait_states(["s_nop 4"]) == 5 and _wait_states(["v_mov_b32 v1, 0", "s_nop 2"]) == 4
+
+
+def test_fp32_kernels_copies_have_their_wait_states(tmp_path):
+    """The fp32 kernels' wave-private copies: the same rules, and M0 written by scalar instructions only."""
+    hipcc = _hipcc()
+    if hipcc is None:
+        pytest.skip("hipcc not available")
+    src, out = tmp_path / "tu.hip", tmp_path / "tu.s"
+    src.write_text('#include "attn_f32_kernels.h"\n' + "".join(
+        f"template __global__ void mt::{k}(mt::AttnParams);\n"
+        for k in ("attn_fwd_f32_kernel<32, true, 4>", "attn_fwd_f32_kernel<64, false, 1>",
+                  "attn_bwd_dq_f32_kernel<128, true, 1>", "attn_bwd_dkv_f32_kernel<64, true>")))
+    proc = subprocess.run([hipcc, "--offload-arch=gfx950", "-O3", "-std=c++17", "--cuda-device-only", "-S",
+                           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-pass-failed",
+                           "-I", CSRC, str(src), "-o", str(out)], capture_output=True, text=True, timeout=900)
+    assert proc.returncode == 0, proc.stderr[-2000:]
+    ins = _instructions(out.read_text())
+    test_every_lds_copy_has_its_wait_states(ins)
+    assert not [x for x in ins if x.startswith("v_") and _writes(x, {"m0"})]

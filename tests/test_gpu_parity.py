@@ -9,6 +9,7 @@ size-independent properties (causality, determinism, GQA expansion).
 
 from __future__ import annotations
 
+import importlib
 import os
 
 import numpy as np
@@ -362,3 +363,44 @@ def test_padded_head_dim_keeps_the_query_layout(mta):
     qv = q.transpose(1, 2).contiguous().to(dev).transpose(1, 2).requires_grad_(True)
     out = mta.attention(qv, k.to(dev), v.to(dev), repeats=2)
     assert out.shape == qv.shape and out.stride() == qv.stride()
+
+
+@pytest.mark.parametrize("b,t,hq,hkv,d", [
+    (1, 1, 2, 1, 32), (2, 31, 3, 1, 64), (2, 32, 4, 4, 128), (1, 33, 4, 2, 64),   # one tile, its edges
+    (1, 129, 7, 1, 32), (3, 160, 2, 2, 128), (1, 257, 6, 2, 64),                  # 5 tiles and more: every wave reuses its LDS block
+    (64, 33, 32, 8, 32), (40, 65, 32, 8, 64), (64, 40, 32, 32, 128),              # enough row blocks for one a wave
+])
+@pytest.mark.parametrize("rope", [False, True])
+def test_fp32_tile_edges_and_both_forward_forms(b, t, hq, hkv, d, rope):
+    """fp32 kernels against float64: ragged tiles, waves without a tile, and grids on both sides of the
+    row-block-per-wave rule (2048 row blocks on a 256-CU GPU).  A value is a sum of at most t + d products
+    of values of the inputs' scale (1), each rounded to 2^-24: the error is at most (t + d) 2^-24 of that scale
+    or of the result where that is larger (at t = 1 dQ and dK cancel to 0); 3e-5 at the largest size here."""
+    g = torch.Generator(device="cuda").manual_seed(t * 100 + d)
+    q, do = (torch.randn(b, t, hq, d, generator=g, device="cuda").transpose(1, 2) for _ in range(2))
+    k, v = (torch.randn(b, t, hkv, d, generator=g, device="cuda").transpose(1, 2) for _ in range(2))
+    ang = torch.outer(torch.arange(t, device="cuda", dtype=torch.float64),
+                      10000.0 ** (-torch.arange(0, d, 2, device="cuda", dtype=torch.float64) / d))
+    cos, sin = ang.cos().float(), ang.sin().float()
+    args = [x.detach().requires_grad_(True) for x in (q, k, v)]
+    mta = importlib.import_module("mega-trading_amd")
+    out = (mta.rope_attention(*args, cos, sin, repeats=hq // hkv) if rope
+           else mta.attention(*args, repeats=hq // hkv))
+    got = (out, *torch.autograd.grad(out, args, do))
+    ref_in = [x.detach().double().requires_grad_(True) for x in (q, k, v)]
+
+    def rot(x):
+        if not rope:
+            return x
+        e, o = x[..., 0::2], x[..., 1::2]
+        c, s = cos.double(), sin.double()
+        return torch.stack((e * c - o * s, e * s + o * c), dim=-1).flatten(-2)
+
+    kk, vv = (x.repeat_interleave(hq // hkv, dim=1) for x in (rot(ref_in[1]), ref_in[2]))
+    s = rot(ref_in[0]) @ kk.transpose(2, 3) / d ** 0.5
+    s = s.masked_fill(torch.ones(t, t, dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+    ref = torch.softmax(s, dim=-1) @ vv
+    refs = (ref, *torch.autograd.grad(ref, ref_in, do.double()))
+    for a, r in zip(got, refs):
+        err = float((a.double() - r).norm() / max(float(r.norm()), r.numel() ** 0.5))
+        assert err <= (t + d) * 2.0 ** -24, err
