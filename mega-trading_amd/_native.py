@@ -11,9 +11,11 @@ import ctypes
 import os
 import threading
 
+import torch
+
 LIB_NAME = "libmt_attn.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
-# the GPU implementations of the mega_trading_amd attention ops (PyTorch-ROCm side, links libmt_attn.so)
+# the GPU implementations and autograd of the mega_trading_amd ops (PyTorch-ROCm side, links libmt_attn.so)
 TORCH_OPS_NAME = "libmt_torch.so"
 TORCH_OPS_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), TORCH_OPS_NAME)
 
@@ -113,7 +115,7 @@ def torch_ops_path() -> str:
 
 def load() -> ctypes.CDLL:
     """Load libmt_attn.so (once) and declare the C signatures; also load
-    libmt_torch.so, which registers the attention ops' GPU kernels with torch."""
+    libmt_torch.so, which registers the ops' GPU kernels and autograd with torch."""
     global _lib
     if _lib is not None:
         return _lib
@@ -127,8 +129,6 @@ def load() -> ctypes.CDLL:
                     "(or python mega-trading_amd/build_lib.py) before using the HIP attention op"
                 )
         lib = ctypes.CDLL(LIB_PATH)
-        import torch
-
         torch.ops.load_library(TORCH_OPS_PATH)
         lib.mt_version.restype = _I
         lib.mt_version.argtypes = []
@@ -150,6 +150,15 @@ def load() -> ctypes.CDLL:
             fn.argtypes = args
         _lib = lib
         return lib
+
+
+@torch.compiler.assume_constant_result
+def ensure() -> bool:
+    """``load()`` for the torch ops' callers: their GPU kernels and autograd
+    formulas are registered (a constant under torch.compile's tracing)."""
+    if _lib is None:
+        load()
+    return True
 
 
 def check(rc: int, what: str) -> None:

@@ -11,8 +11,8 @@ the kernels' Q/K tile loads.
 
 The attention ops are ``torch.library`` ops (``mega_trading_amd::gqa_attn_fwd``,
 ``::gqa_rope_attn_fwd``, ``::gqa_attn_bwd`` and the packed q|k|v pair) whose
-schemas, fake implementations and autograd are declared here, so
-``torch.compile`` treats them as opaque nodes; their GPU implementations live
+schemas and fake implementations are declared here, so ``torch.compile``
+treats them as opaque nodes; their autograd and GPU implementations live
 in ``libmt_torch.so`` (``csrc/mt_torch.cpp``), which prepares the arguments,
 allocates the outputs and calls the C ABI of ``libmt_attn.so`` on the
 caller's current stream.  They never synchronise and never fall back to
@@ -109,8 +109,8 @@ def rope_attention_packed(
     d = q.shape[-1]
     if d not in KERNEL_HEAD_DIMS:
         raise ValueError(f"the packed form needs head_dim {KERNEL_HEAD_DIMS} (got {d}); use rope_attention")
-    _native.load()
-    out, _lse, _q_rot, _k_rot = torch.ops.mega_trading_amd.gqa_rope_attn_packed_fwd(
+    _native.ensure()
+    out, _lse, _q_rot, _k_rot = _rope_attn_packed_fwd(
         qkv, c, s, heads, kv_heads, 1.0 / math.sqrt(d))
     return out
 
@@ -187,6 +187,7 @@ def decode_attention(
     if query.shape[-1] not in KERNEL_HEAD_DIMS:
         raise ValueError(f"head_dim must be one of {KERNEL_HEAD_DIMS} (got {query.shape[-1]})")
     scale = 1.0 / math.sqrt(query.shape[-1])
+    _native.ensure()
     if repeats > MAX_DECODE_REPEATS:
         # the group's query heads in even sub-groups of at most MAX_DECODE_REPEATS,
         # each one launch over the same cache (a sub-group is a GQA group of its own)
@@ -200,8 +201,8 @@ def decode_attention(
                  for lo, hi in zip(bounds[:-1], bounds[1:])]
         return torch.cat(parts, dim=2).view(b, hq, 1, d)
     if dev_length:
-        return torch.ops.mega_trading_amd.gqa_attn_decode_dev(query, key_cache, value_cache, length, scale)
-    return torch.ops.mega_trading_amd.gqa_attn_decode(query, key_cache, value_cache, int(length), scale)
+        return _attn_decode_dev(query, key_cache, value_cache, length, scale)
+    return _attn_decode(query, key_cache, value_cache, int(length), scale)
 
 
 def decode_rope_append(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, cos: torch.Tensor,
@@ -217,10 +218,11 @@ def decode_rope_append(query: torch.Tensor, key: torch.Tensor, value: torch.Tens
     last = _check_append(query, key, value, cos, sin, pos, key_cache, value_cache)
     # the kernel reads fp32 tables (a model cast with .to(dtype) casts its RoPE buffers too)
     cos, sin = cos.to(torch.float32), sin.to(torch.float32)
+    _native.ensure()
     if isinstance(pos, torch.Tensor):
-        return torch.ops.mega_trading_amd.decode_rope_append(query, key, value, cos, sin, last, pos, key_cache,
+        return _rope_append(query, key, value, cos, sin, last, pos, key_cache,
                                                              value_cache)
-    return torch.ops.mega_trading_amd.decode_rope_append(query, key, value, cos, sin, int(pos), None, key_cache,
+    return _rope_append(query, key, value, cos, sin, int(pos), None, key_cache,
                                                          value_cache)
 
 
@@ -283,12 +285,13 @@ def decode_append_attention(query: torch.Tensor, key: torch.Tensor, value: torch
     if key_cache.shape[1] * repeats != hq or key_cache.shape[0] != b:
         raise ValueError("query heads must equal key/value heads multiplied by repeats")
     scale = 1.0 / math.sqrt(d)
+    _native.ensure()
     if dev:
         if length.dtype != torch.int32 or length.numel() != 1 or length.device != query.device:
             raise ValueError("a tensor length must be a one-element int32 tensor on the query's device")
-        return torch.ops.mega_trading_amd.gqa_attn_decode_append(query, key, value, cos, sin, last, pos, 0, length,
+        return _attn_decode_append(query, key, value, cos, sin, last, pos, 0, length,
                                                                  key_cache, value_cache, scale)
-    return torch.ops.mega_trading_amd.gqa_attn_decode_append(query, key, value, cos, sin, int(pos), None, int(length),
+    return _attn_decode_append(query, key, value, cos, sin, int(pos), None, int(length),
                                                              None, key_cache, value_cache, scale)
 
 
@@ -326,10 +329,13 @@ def _rope_tables(cos: torch.Tensor, sin: torch.Tensor, query: torch.Tensor) -> t
     for name, tab in (("cos", cos), ("sin", sin)):
         if tab.shape[-1] != d // 2:
             raise ValueError(f"RoPE {name} table must have last dimension head_dim/2 = {d // 2}")
-        tab2 = tab.reshape(-1, d // 2)
-        if tab2.shape[0] < t:
-            raise ValueError(f"sequence length {t} exceeds RoPE cache length {tab2.shape[0]}")
-        out.append(tab2[:t].to(device=query.device, dtype=torch.float32).contiguous())
+        rows = tab.numel() // (d // 2)
+        if rows < t:
+            raise ValueError(f"sequence length {t} exceeds RoPE cache length {rows}")
+        if tab.dtype == torch.float32 and tab.device == query.device and tab.is_contiguous():
+            out.append(tab)  # as RotaryEmbedding keeps it: the kernels read its first t rows
+        else:
+            out.append(tab.reshape(-1, d // 2)[:t].to(device=query.device, dtype=torch.float32).contiguous())
     return out[0], out[1]
 
 
@@ -366,11 +372,11 @@ def _forward(q, k, v, cos, sin):
     dk = _kernel_head_dim(d)
     if dk != d:
         return _forward_padded(q, k, v, cos, sin, dk)
-    _native.load()
+    _native.ensure()
     scale = 1.0 / math.sqrt(d)
     if cos is None:
-        return torch.ops.mega_trading_amd.gqa_attn_fwd(q, k, v, scale)
-    out, lse, _q_rot, _k_rot = torch.ops.mega_trading_amd.gqa_rope_attn_fwd(q, k, v, cos, sin, scale)
+        return _attn_fwd(q, k, v, scale)
+    out, lse, _q_rot, _k_rot = _rope_attn_fwd(q, k, v, cos, sin, scale)
     return out, lse
 
 
@@ -385,15 +391,15 @@ def _forward_padded(q, k, v, cos, sin, dk):
     d = q.shape[-1]
     pad = (0, dk - d)
     qp, kp, vp = F.pad(q, pad), F.pad(k, pad), F.pad(v, pad)
-    _native.load()
+    _native.ensure()
     scale = 1.0 / math.sqrt(d)
     if cos is None:
-        out, lse = torch.ops.mega_trading_amd.gqa_attn_fwd(qp, kp, vp, scale)
+        out, lse = _attn_fwd(qp, kp, vp, scale)
     else:
         half = (dk - d) // 2
         cos = F.pad(cos, (0, half), value=1.0)
         sin = F.pad(sin, (0, half), value=0.0)
-        out, lse, _q_rot, _k_rot = torch.ops.mega_trading_amd.gqa_rope_attn_fwd(qp, kp, vp, cos, sin, scale)
+        out, lse, _q_rot, _k_rot = _rope_attn_fwd(qp, kp, vp, cos, sin, scale)
     result = torch.empty_like(q)
     result.copy_(out[..., :d])
     return result, lse
@@ -453,167 +459,41 @@ def _gqa_attn_bwd_packed_fake(q_rot, k_rot, qkv, out, lse, dout, cos, sin, hq, h
     return qkv.new_empty(qkv.shape)
 
 
-@torch.library.custom_op("mega_trading_amd::gqa_attn_decode", mutates_args=(), device_types="cuda")
-def gqa_attn_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, length: int,
-                    scale: float) -> torch.Tensor:
-    lib = _native.load()
-    q, k_cache, v_cache = _kernel_ready(q), _kernel_ready(k_cache), _kernel_ready(v_cache)
-    b, hq, _, d = q.shape
-    hkv = k_cache.shape[1]
-    out = torch.empty((b, hq, 1, d), device=q.device, dtype=q.dtype)
-    strides = _strides(q, k_cache, v_cache, out)
-    with torch.cuda.device(q.device):
-        ws_bytes = lib.mt_gqa_attn_decode_workspace_size(b, hq, length, d)
-        ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)
-        rc = lib.mt_gqa_attn_decode(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), b, hq, hkv,
-                                    length, d, strides, scale, _KERNEL_DTYPES[q.dtype], ws.data_ptr(), ws_bytes,
-                                    torch.cuda.current_stream(q.device).cuda_stream)
-    _native.check(rc, "mt_gqa_attn_decode")
-    return out
+_LIB.define("gqa_attn_decode(Tensor q, Tensor k_cache, Tensor v_cache, SymInt length, float scale) -> Tensor")
+_LIB.define("gqa_attn_decode_dev(Tensor q, Tensor k_cache, Tensor v_cache, Tensor length, float scale) -> Tensor")
+_LIB.define("decode_rope_append(Tensor q, Tensor k, Tensor v, Tensor cos, Tensor sin, SymInt pos, Tensor? pos_dev, "
+            "Tensor(a!) k_cache, Tensor(b!) v_cache) -> Tensor")
+_LIB.define("gqa_attn_decode_append(Tensor q, Tensor k, Tensor v, Tensor cos, Tensor sin, SymInt pos, "
+            "Tensor? pos_dev, SymInt length, Tensor? length_dev, Tensor(a!) k_cache, Tensor(b!) v_cache, float scale) "
+            "-> Tensor")
 
 
-@torch.library.custom_op("mega_trading_amd::decode_rope_append", mutates_args=("k_cache", "v_cache"),
-                         device_types="cuda")
-def decode_rope_append_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
-                          pos: int, pos_dev: Optional[torch.Tensor], k_cache: torch.Tensor,
-                          v_cache: torch.Tensor) -> torch.Tensor:
-    import ctypes
-
-    lib = _native.load()
-    b, hq, _, d = q.shape
-    hkv = k.shape[1]
-    q_rot = torch.empty((b, hq, 1, d), device=q.device, dtype=k_cache.dtype)
-    cs = cos.reshape(-1, d // 2).contiguous()
-    sn = sin.reshape(-1, d // 2).contiguous()
-    ins = (ctypes.c_int64 * 6)(q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1))
-    cst = (ctypes.c_int64 * 6)(*k_cache.stride()[:3], *v_cache.stride()[:3])
-    in_dt = _native.DTYPE_FP32 if q.dtype == torch.float32 else _KERNEL_DTYPES[q.dtype]
-    with torch.cuda.device(q.device):
-        rc = lib.mt_decode_rope_append(q.data_ptr(), k.data_ptr(), v.data_ptr(), ins, cs.data_ptr(), sn.data_ptr(),
-                                       min(cs.shape[0], sn.shape[0]), pos, _ptr(pos_dev), q_rot.data_ptr(),
-                                       k_cache.data_ptr(), v_cache.data_ptr(), cst, k_cache.shape[2],
-                                       b, hq, hkv, d,
-                                       in_dt, _KERNEL_DTYPES[k_cache.dtype],
-                                       torch.cuda.current_stream(q.device).cuda_stream)
-    _native.check(rc, "mt_decode_rope_append")
-    return q_rot
-
-
-@decode_rope_append_op.register_fake
+@torch.library.register_fake("mega_trading_amd::decode_rope_append")
 def _decode_rope_append_fake(q, k, v, cos, sin, pos, pos_dev, k_cache, v_cache):
     return q.new_empty(q.shape, dtype=k_cache.dtype)
 
 
-@torch.library.custom_op("mega_trading_amd::gqa_attn_decode_dev", mutates_args=(), device_types="cuda")
-def gqa_attn_decode_dev(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, length: torch.Tensor,
-                        scale: float) -> torch.Tensor:
-    lib = _native.load()
-    q, k_cache, v_cache = _kernel_ready(q), _kernel_ready(k_cache), _kernel_ready(v_cache)
-    b, hq, _, d = q.shape
-    hkv, cap = k_cache.shape[1], k_cache.shape[2]
-    out = torch.empty((b, hq, 1, d), device=q.device, dtype=q.dtype)
-    strides = _strides(q, k_cache, v_cache, out)
-    with torch.cuda.device(q.device):
-        ws_bytes = lib.mt_gqa_attn_decode_workspace_size(b, hq, cap, d)
-        ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)
-        rc = lib.mt_gqa_attn_decode_dev(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), b, hq,
-                                        hkv, cap, length.data_ptr(), d, strides, scale, _KERNEL_DTYPES[q.dtype],
-                                        ws.data_ptr(), ws_bytes, torch.cuda.current_stream(q.device).cuda_stream)
-    _native.check(rc, "mt_gqa_attn_decode_dev")
-    return out
-
-
-@torch.library.custom_op("mega_trading_amd::gqa_attn_decode_append", mutates_args=("k_cache", "v_cache"),
-                         device_types="cuda")
-def gqa_attn_decode_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
-                           pos: int, pos_dev: Optional[torch.Tensor], length: int, length_dev: Optional[torch.Tensor],
-                           k_cache: torch.Tensor, v_cache: torch.Tensor, scale: float) -> torch.Tensor:
-    import ctypes
-
-    lib = _native.load()
-    b, hq, _, d = q.shape
-    hkv, cap = k_cache.shape[1], k_cache.shape[2]
-    out = torch.empty((b, hq, 1, d), device=q.device, dtype=k_cache.dtype)
-    ins = (ctypes.c_int64 * 6)(q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1))
-    cst = (ctypes.c_int64 * 6)(*k_cache.stride()[:3], *v_cache.stride()[:3])
-    in_dt = _native.DTYPE_FP32 if q.dtype == torch.float32 else _KERNEL_DTYPES[q.dtype]
-    with torch.cuda.device(q.device):
-        ws_bytes = lib.mt_gqa_attn_decode_workspace_size(b, hq, cap if length_dev is not None else max(length, pos + 1), d)
-        ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)
-        rc = lib.mt_gqa_attn_decode_append(q.data_ptr(), k.data_ptr(), v.data_ptr(), ins, cos.data_ptr(), sin.data_ptr(),
-                                           cos.numel() // (d // 2), pos, _ptr(pos_dev), k_cache.data_ptr(),
-                                           v_cache.data_ptr(), cst, cap, length, _ptr(length_dev), out.data_ptr(), b, hq,
-                                           hkv, d, scale, in_dt, _KERNEL_DTYPES[k_cache.dtype], ws.data_ptr(), ws_bytes,
-                                           torch.cuda.current_stream(q.device).cuda_stream)
-    _native.check(rc, "mt_gqa_attn_decode_append")
-    return out
-
-
-@gqa_attn_decode_append.register_fake
+@torch.library.register_fake("mega_trading_amd::gqa_attn_decode_append")
 def _gqa_attn_decode_append_fake(q, k, v, cos, sin, pos, pos_dev, length, length_dev, k_cache, v_cache, scale):
     return q.new_empty(q.shape, dtype=k_cache.dtype)
 
 
-@gqa_attn_decode_dev.register_fake
+@torch.library.register_fake("mega_trading_amd::gqa_attn_decode_dev")
 def _gqa_attn_decode_dev_fake(q, k_cache, v_cache, length, scale):
     return q.new_empty(q.shape)
 
 
-@gqa_attn_decode.register_fake
+@torch.library.register_fake("mega_trading_amd::gqa_attn_decode")
 def _gqa_attn_decode_fake(q, k_cache, v_cache, length, scale):
     return q.new_empty(q.shape)
 
 
-def _fwd_setup_context(ctx, inputs, output):
-    q, k, v, scale = inputs
-    out, lse = output
-    ctx.save_for_backward(q, k, v, out, lse)
-    ctx.scale = scale
-    ctx.mark_non_differentiable(lse)
-    ctx.set_materialize_grads(False)
-
-
-def _fwd_backward(ctx, grad_out, _grad_lse):
-    q, k, v, out, lse = ctx.saved_tensors
-    dq, dk, dv = torch.ops.mega_trading_amd.gqa_attn_bwd(q, k, v, out, lse, grad_out, None, None, ctx.scale)
-    return dq, dk, dv, None
-
-
-def _rope_fwd_setup_context(ctx, inputs, output):
-    _q, _k, v, cos, sin, scale = inputs
-    out, lse, q_rot, k_rot = output
-    ctx.save_for_backward(q_rot, k_rot, v, out, lse, cos, sin)
-    ctx.scale = scale
-    ctx.mark_non_differentiable(lse, q_rot, k_rot)
-    ctx.set_materialize_grads(False)
-
-
-def _rope_fwd_backward(ctx, grad_out, _grad_lse, _grad_q_rot, _grad_k_rot):
-    q_rot, k_rot, v, out, lse, cos, sin = ctx.saved_tensors
-    dq, dk, dv = torch.ops.mega_trading_amd.gqa_attn_bwd(q_rot, k_rot, v, out, lse, grad_out, cos, sin, ctx.scale)
-    return dq, dk, dv, None, None, None
-
-
-def _packed_setup_context(ctx, inputs, output):
-    qkv, cos, sin, hq, hkv, scale = inputs
-    out, lse, q_rot, k_rot = output
-    ctx.save_for_backward(q_rot, k_rot, qkv, out, lse, cos, sin)
-    ctx.hq, ctx.hkv, ctx.scale = hq, hkv, scale
-    ctx.mark_non_differentiable(lse, q_rot, k_rot)
-    ctx.set_materialize_grads(False)
-
-
-def _packed_backward(ctx, grad_out, _grad_lse, _grad_q_rot, _grad_k_rot):
-    if grad_out is None:
-        return None, None, None, None, None, None
-    q_rot, k_rot, qkv, out, lse, cos, sin = ctx.saved_tensors
-    dqkv = torch.ops.mega_trading_amd.gqa_attn_bwd_packed(q_rot, k_rot, qkv, out, lse, grad_out, cos, sin, ctx.hq,
-                                                          ctx.hkv, ctx.scale)
-    return dqkv, None, None, None, None, None
-
-
-torch.library.register_autograd("mega_trading_amd::gqa_attn_fwd", _fwd_backward, setup_context=_fwd_setup_context)
-torch.library.register_autograd("mega_trading_amd::gqa_rope_attn_packed_fwd", _packed_backward,
-                                setup_context=_packed_setup_context)
-torch.library.register_autograd("mega_trading_amd::gqa_rope_attn_fwd", _rope_fwd_backward,
-                                setup_context=_rope_fwd_setup_context)
+# the ops as the functions above call them
+_OPS = torch.ops.mega_trading_amd
+_attn_fwd = _OPS.gqa_attn_fwd.default
+_rope_attn_fwd = _OPS.gqa_rope_attn_fwd.default
+_rope_attn_packed_fwd = _OPS.gqa_rope_attn_packed_fwd.default
+_attn_decode = _OPS.gqa_attn_decode.default
+_attn_decode_dev = _OPS.gqa_attn_decode_dev.default
+_rope_append = _OPS.decode_rope_append.default
+_attn_decode_append = _OPS.gqa_attn_decode_append.default

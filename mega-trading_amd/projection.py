@@ -30,7 +30,6 @@ Backward:
 
 from __future__ import annotations
 
-import ctypes
 from typing import Optional, Sequence
 
 import torch
@@ -136,49 +135,34 @@ def _rows_path(x2: torch.Tensor, weights: Sequence[torch.Tensor], dtype: torch.d
                and w.data_ptr() % 16 == 0 for w in weights)
 
 
-@torch.library.custom_op("mega_trading_amd::linear_rows", mutates_args=(), device_types="cuda")
-def linear_rows(x: torch.Tensor, weights: list[torch.Tensor]) -> torch.Tensor:
+_LIB = torch.library.Library("mega_trading_amd", "FRAGMENT")
+_LIB.define("linear_rows(Tensor x, Tensor[] weights) -> Tensor")
+_LIB.define("linear_rows_gate(Tensor x, Tensor w_gate, Tensor w_up) -> Tensor")
+
+
+def linear_rows(x: torch.Tensor, weights: Sequence[torch.Tensor]) -> torch.Tensor:
     """[rows, sum(out_i)] = cat([x.float() @ w.T for w in weights], -1), fp32,
     for x [rows <= 64, K] (fp32 or 16-bit) and fp32 weights [out_i, K]
     (``mt_linear_rows``)."""
-    lib = _native.load()
-    rows, k = x.shape
-    outs = [w.shape[0] for w in weights]
-    y = torch.empty((rows, sum(outs)), device=x.device, dtype=torch.float32)
-    g = len(weights)
-    ptrs = (ctypes.c_void_p * g)(*[w.data_ptr() for w in weights])
-    ns = (ctypes.c_int * g)(*outs)
-    lds = (ctypes.c_int64 * g)(*[w.stride(0) for w in weights])
-    with torch.cuda.device(x.device):
-        rc = lib.mt_linear_rows(x.data_ptr(), x.stride(0), ptrs, ns, lds, g, y.data_ptr(), y.stride(0), rows, k,
-                                _X_DTYPES[x.dtype], torch.cuda.current_stream(x.device).cuda_stream)
-    _native.check(rc, "mt_linear_rows")
-    return y
+    _native.ensure()
+    return torch.ops.mega_trading_amd.linear_rows.default(x, list(weights))
 
 
-@torch.library.custom_op("mega_trading_amd::linear_rows_gate", mutates_args=(), device_types="cuda")
 def linear_rows_gate(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor) -> torch.Tensor:
     """silu(x @ w_gate.T) * (x @ w_up.T) [rows, out], fp32, for x and the
     weights as ``linear_rows`` takes them (``mt_linear_rows_gate``)."""
-    lib = _native.load()
-    rows, k = x.shape
-    y = torch.empty((rows, w_gate.shape[0]), device=x.device, dtype=torch.float32)
-    with torch.cuda.device(x.device):
-        rc = lib.mt_linear_rows_gate(x.data_ptr(), x.stride(0), w_gate.data_ptr(), w_up.data_ptr(), w_gate.stride(0),
-                                     w_up.stride(0), y.data_ptr(), y.stride(0), rows, k, w_gate.shape[0],
-                                     _X_DTYPES[x.dtype], torch.cuda.current_stream(x.device).cuda_stream)
-    _native.check(rc, "mt_linear_rows_gate")
-    return y
+    _native.ensure()
+    return torch.ops.mega_trading_amd.linear_rows_gate.default(x, w_gate, w_up)
 
 
-@linear_rows_gate.register_fake
+@torch.library.register_fake("mega_trading_amd::linear_rows_gate")
 def _linear_rows_gate_fake(x, w_gate, w_up):
     return x.new_empty((x.shape[0], w_gate.shape[0]), dtype=torch.float32)
 
 
-@linear_rows.register_fake
+@torch.library.register_fake("mega_trading_amd::linear_rows")
 def _linear_rows_fake(x, weights):
-    return x.new_empty((x.shape[0], sum(w.shape[0] for w in weights)))
+    return x.new_empty((x.shape[0], sum(w.shape[0] for w in weights)), dtype=torch.float32)
 
 
 def _check(x: torch.Tensor, weights: Sequence[torch.Tensor]) -> None:
@@ -198,7 +182,7 @@ def project_packed(x: torch.Tensor, weights: Sequence[torch.Tensor]) -> torch.Te
     dtype = _compute_dtype(x, weights)
     x2 = x.reshape(-1, x.shape[-1])
     if _rows_path(x2, weights, dtype):
-        return linear_rows(x2, list(weights)).view(*x.shape[:-1], -1)
+        return linear_rows(x2, weights).view(*x.shape[:-1], -1)
     return _Project.apply(x, dtype, *weights)
 
 
