@@ -35,6 +35,31 @@ constexpr int kDtFP32 = 2;
 // ---------------------------------------------------------------------------
 template <int DT>
 struct IO {
+  // 8 values as loaded (unpacked only where they are used: half the registers
+  // of a 16-bit row while it is in flight)
+  struct Raw {
+    u32x4 w[DT == kDtFP32 ? 2 : 1];
+  };
+  static __device__ __forceinline__ Raw load_raw(const void* base, int64_t i) {
+    Raw r;
+    const u32x4* p = reinterpret_cast<const u32x4*>(static_cast<const char*>(base) + i * (DT == kDtFP32 ? 4 : 2));
+    r.w[0] = p[0];
+    if constexpr (DT == kDtFP32) r.w[1] = p[1];
+    return r;
+  }
+  static __device__ __forceinline__ void unpack(const Raw& r, float* v) {
+    if constexpr (DT == kDtFP32) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = __uint_as_float(r.w[k >> 2][k & 3]);
+    } else {
+      using E = typename std::conditional<DT == kDtBF16, BF16, FP16>::type;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        v[2 * k] = lo_f<E>(r.w[0][k]);
+        v[2 * k + 1] = hi_f<E>(r.w[0][k]);
+      }
+    }
+  }
   static __device__ __forceinline__ void load8(const void* base, int64_t i, float* v) {
     if constexpr (DT == kDtFP32) {
       const f32x4* p = reinterpret_cast<const f32x4*>(static_cast<const float*>(base) + i);
@@ -164,7 +189,33 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const void* x, int64_t
 // gradient of a 16-bit branch input of the mixed add).  Waves stride over
 // rows; each lane accumulates its dw chunks in registers, the 4 waves of a
 // workgroup combine them in LDS and write one fp32 partial row per workgroup.
+// Bound by memory: a wave holds its next row in flight while it works on the
+// current one, every input of the row asked for at once (d_new_res used to be
+// loaded behind the row sum).  Residual form, forward +
+// backward, bf16: 32768 x 1024 112.6 -> 102.9 us, 15000 x 4096 332 -> 213; fp32
+// 9000 x 4096 253 -> 246, 32768 x 512 unchanged (101).
 // ===========================================================================
+template <int ST, int GT, int NCH, bool D_TOO>
+struct NormBwdRow {
+  typename IO<ST>::Raw s[NCH], d[D_TOO ? NCH : 1];
+  typename IO<GT>::Raw g[NCH];
+  float rstd;
+  __device__ __forceinline__ void load(const void* sp, const float* rp, const void* gp, const void* dp, int64_t row,
+                                       int64_t rows, int D, int lane, int nch) {
+    if (row >= rows) return;  // (wave-uniform)
+    rstd = rp[row];
+#pragma unroll
+    for (int k = 0; k < NCH; ++k) {
+      const int c = lane + 64 * k;
+      if (c < nch) {
+        s[k] = IO<ST>::load_raw(sp, row * D + 8 * c);
+        g[k] = IO<GT>::load_raw(gp, row * D + 8 * c);
+        if constexpr (D_TOO) d[k] = IO<ST>::load_raw(dp, row * D + 8 * c);
+      }
+    }
+  }
+};
+
 template <int ST, int GT, int WT, int NCH, bool ADD>
 __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const void* s, const void* w, const float* rstd,
                                                           const void* dy, const void* dres, void* ds, void* ds16,
@@ -182,64 +233,54 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const void* s, const v
     for (int j = 0; j < 8; ++j) acc[k][j] = 0.f;
     if (c < nch) IO<WT>::load8(w, 8 * c, wv[k]);
   }
-  // U rows per iteration, all loads issued before any arithmetic, so each wave
-  // keeps U rows of traffic in flight
-  constexpr int U = NCH <= 2 ? 2 : 1;
+  // two rows' registers where they fit; the widest fp32 rows keep d_new_res for
+  // its use (2000 x 1768: 31.7 us with it held, 30.1 without)
+  constexpr bool AHEAD = NCH * (ST == kDtFP32 ? 2 : 1) <= 4;
+  constexpr bool D_TOO = ADD && (AHEAD || ST != kDtFP32);
   const int64_t waves = (int64_t)gridDim.x * 4;
-  for (int64_t row0 = (int64_t)blockIdx.x * 4 + wave; row0 < rows; row0 += U * waves) {
-    float sv[U][NCH][8], g[U][NCH][8], r[U];
+  int64_t row = (int64_t)blockIdx.x * 4 + wave;
+  NormBwdRow<ST, GT, NCH, D_TOO> cur, next;
+  if constexpr (AHEAD) cur.load(s, rstd, dy, dres, row, rows, D, lane, nch);
+  for (; row < rows; row += waves) {
+    if constexpr (AHEAD) next.load(s, rstd, dy, dres, row + waves, rows, D, lane, nch);
+    else cur.load(s, rstd, dy, dres, row, rows, D, lane, nch);
+    float sv[NCH][8], g[NCH][8];
+    const float r = cur.rstd;
+    float cs = 0.f;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t row = row0 + u * waves;
-      if (row < rows) {
-        r[u] = rstd[row];
+    for (int k = 0; k < NCH; ++k) {
+      if (lane + 64 * k < nch) {
+        IO<ST>::unpack(cur.s[k], sv[k]);
+        IO<GT>::unpack(cur.g[k], g[k]);
 #pragma unroll
-        for (int k = 0; k < NCH; ++k) {
-          const int c = lane + 64 * k;
-          if (c < nch) {
-            IO<ST>::load8(s, row * D + 8 * c, sv[u][k]);
-            IO<GT>::load8(dy, row * D + 8 * c, g[u][k]);
-          }
+        for (int j = 0; j < 8; ++j) {
+          acc[k][j] += g[k][j] * sv[k][j] * r;
+          g[k][j] *= wv[k][j];
+          cs += g[k][j] * sv[k][j];
         }
       }
     }
+    cs = wave_sum(cs);
+    const float f = r * r * inv_d * cs;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t row = row0 + u * waves;
-      if (row >= rows) break;
-      float cs = 0.f;
+    for (int k = 0; k < NCH; ++k) {
+      const int c = lane + 64 * k;
+      if (c < nch) {
+        float o[8];
 #pragma unroll
-      for (int k = 0; k < NCH; ++k) {
-        const int c = lane + 64 * k;
-        if (c < nch) {
+        for (int j = 0; j < 8; ++j) o[j] = r * (g[k][j] - sv[k][j] * f);
+        if constexpr (ADD) {
+          float dr[8];
+          if constexpr (D_TOO) IO<ST>::unpack(cur.d[k], dr);
+          else IO<ST>::load8(dres, row * D + 8 * c, dr);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            acc[k][j] += g[u][k][j] * sv[u][k][j] * r[u];
-            g[u][k][j] *= wv[k][j];
-            cs += g[u][k][j] * sv[u][k][j];
-          }
+          for (int j = 0; j < 8; ++j) o[j] += dr[j];
         }
-      }
-      cs = wave_sum(cs);
-      const float f = r[u] * r[u] * inv_d * cs;
-#pragma unroll
-      for (int k = 0; k < NCH; ++k) {
-        const int c = lane + 64 * k;
-        if (c < nch) {
-          float o[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) o[j] = r[u] * (g[u][k][j] - sv[u][k][j] * f);
-          if constexpr (ADD) {
-            float dr[8];
-            IO<ST>::load8(dres, row * D + 8 * c, dr);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) o[j] += dr[j];
-          }
-          IO<ST>::store8(ds, row * D + 8 * c, o);
-          if (ds16) IO<GT>::store8(ds16, row * D + 8 * c, o);
-        }
+        IO<ST>::store8(ds, row * D + 8 * c, o);
+        if (ds16) IO<GT>::store8(ds16, row * D + 8 * c, o);
       }
     }
+    if constexpr (AHEAD) cur = next;
   }
   // workgroup reduction of dw: waves 1..3 park their sums, wave 0 adds them
   if (wave > 0) {
