@@ -155,6 +155,16 @@ int mt_cross_entropy_rows(void* logits, int64_t row_stride, const int64_t* label
                           const int64_t* n_valid, int64_t ignore_index, float* loss_rows, int write_grad, int dtype,
                           void* stream);
 
+/* The scalars of a loss head, rows <= 131072, in one launch each: *n_valid = the
+ * number of labels != ignore_index, *loss = the sum of loss_rows (a fixed order).
+ * mt_scale_pair: a_out = a * s and b_out = b * s for two contiguous tensors, s =
+ * *scale rounded to each tensor's type (as torch's product with a scalar tensor of
+ * that type); pointers 16-byte aligned, outputs may be the inputs. */
+int mt_cross_entropy_count(const int64_t* labels, int64_t rows, int64_t ignore_index, int64_t* n_valid, void* stream);
+int mt_cross_entropy_sum(const float* loss_rows, int64_t rows, float* loss, void* stream);
+int mt_scale_pair(const void* a, void* a_out, int64_t na, int a_dtype, const void* b, void* b_out, int64_t nb, int b_dtype,
+                  const float* scale, void* stream);
+
 /* Stand-alone RoPE of q [B, Hq, T, D] and k [B, Hkv, T, D]: each
  * interleaved pair (x[2i], x[2i+1]) = (e, o) of row t becomes
  *   (e c - o s, e s + o c),  c = rope_cos[t * table_stride + i], s = rope_sin[...]

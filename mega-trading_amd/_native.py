@@ -49,6 +49,9 @@ EXPORTS = (
     "mt_swiglu_packed_fwd",
     "mt_swiglu_packed_bwd",
     "mt_cross_entropy_rows",
+    "mt_cross_entropy_count",
+    "mt_cross_entropy_sum",
+    "mt_scale_pair",
     "mt_apply_rope",
     "mt_gqa_attn_decode_workspace_size",
     "mt_gqa_attn_decode",
@@ -87,6 +90,9 @@ _OPS_SIGNATURES = {
     "mt_swiglu_packed_fwd": (_I, [_P, _P, _L, _L, _I, _P]),
     "mt_swiglu_packed_bwd": (_I, [_P, _P, _P, _L, _L, _I, _P]),
     "mt_cross_entropy_rows": (_I, [_P, _L, _P, _L, _I, _P, _L, _P, _I, _I, _P]),
+    "mt_cross_entropy_count": (_I, [_P, _L, _L, _P, _P]),
+    "mt_cross_entropy_sum": (_I, [_P, _L, _P, _P]),
+    "mt_scale_pair": (_I, [_P, _P, _L, _I, _P, _P, _L, _I, _P, _P]),
     "mt_apply_rope": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _L, _I, _I, _I, _P]),
     "mt_gqa_attn_decode_workspace_size": (_S, [_I, _I, _I, _I]),
     "mt_gqa_attn_decode": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _F, _I, _P, _S, _P]),

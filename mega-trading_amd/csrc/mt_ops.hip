@@ -477,6 +477,48 @@ int mt_cross_entropy_rows(void* logits, int64_t row_stride, const int64_t* label
   return e == hipSuccess ? ok() : fail((int)e, "launch failed: %s", hipGetErrorString(e));
 }
 
+int mt_cross_entropy_count(const int64_t* labels, int64_t rows, int64_t ignore_index, int64_t* n_valid, void* stream) {
+  if (rows < 0 || rows > K::kCeScalarRows)
+    return fail(MT_E_SHAPE, "rows must be in [0, %lld] (got %lld)", (long long)K::kCeScalarRows, (long long)rows);
+  if ((rows && !labels) || !n_valid) return fail(MT_E_NULL, "labels or n_valid is NULL");
+  hipLaunchKernelGGL(K::ce_count_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, labels, rows, ignore_index, n_valid);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? ok() : fail((int)e, "launch failed: %s", hipGetErrorString(e));
+}
+
+int mt_cross_entropy_sum(const float* loss_rows, int64_t rows, float* loss, void* stream) {
+  if (rows < 0 || rows > K::kCeScalarRows)
+    return fail(MT_E_SHAPE, "rows must be in [0, %lld] (got %lld)", (long long)K::kCeScalarRows, (long long)rows);
+  if ((rows && !loss_rows) || !loss) return fail(MT_E_NULL, "loss_rows or loss is NULL");
+  hipLaunchKernelGGL(K::ce_sum_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, loss_rows, rows, loss);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? ok() : fail((int)e, "launch failed: %s", hipGetErrorString(e));
+}
+
+int mt_scale_pair(const void* a, void* a_out, int64_t na, int a_dtype, const void* b, void* b_out, int64_t nb, int b_dtype,
+                  const float* scale, void* stream) {
+  int rc;
+  if ((rc = check_dtype(a_dtype, a_dtype)) || (rc = check_dtype(b_dtype, b_dtype))) return rc;
+  if (na < 0 || nb < 0) return fail(MT_E_SHAPE, "sizes must be >= 0 (got %lld, %lld)", (long long)na, (long long)nb);
+  if (na + nb == 0) return ok();
+  if (!scale) return fail(MT_E_NULL, "scale is NULL");
+  if (na && ((rc = check_ptr("a", a)) || (rc = check_ptr("a_out", a_out)))) return rc;
+  if (nb && ((rc = check_ptr("b", b)) || (rc = check_ptr("b_out", b_out)))) return rc;
+  const int64_t chunks = (na + 7) / 8 + (nb + 7) / 8, want = (chunks + 255) / 256, cap = 16L * device_cus();
+  const dim3 grid((unsigned)(want < cap ? want : cap));
+  hipStream_t st = (hipStream_t)stream;
+#define MT_SCALE(A, B) \
+  if (a_dtype == A && b_dtype == B) hipLaunchKernelGGL((K::scale_pair_kernel<A, B>), grid, dim3(256), 0, st, a, a_out, na, b, b_out, nb, scale)
+#define MT_SCALE_A(A) MT_SCALE(A, 0); MT_SCALE(A, 1); MT_SCALE(A, 2)
+  MT_SCALE_A(0);
+  MT_SCALE_A(1);
+  MT_SCALE_A(2);
+#undef MT_SCALE_A
+#undef MT_SCALE
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? ok() : fail((int)e, "launch failed: %s", hipGetErrorString(e));
+}
+
 int mt_apply_rope(const void* q, const void* k, void* q_out, void* k_out, int B, int Hq, int Hkv, int T, int D,
                   const int64_t* strides, const float* rope_cos, const float* rope_sin, int64_t table_stride,
                   int table_rows, int inverse, int dtype, void* stream) {

@@ -505,6 +505,35 @@ at::Tensor linear_rows_gate(const at::Tensor& x, const at::Tensor& w_gate, const
   return y;
 }
 
+// --- loss head (schemas in ops.py; the op itself, which runs library GEMMs, is Python) ---
+at::Tensor ce_count(const at::Tensor& labels, int64_t ignore_index) {
+  const c10::DeviceGuard guard(labels.device());
+  const at::Tensor n = at::empty({}, labels.options());
+  check_rc(mt_cross_entropy_count(static_cast<const int64_t*>(labels.data_ptr()), labels.numel(), ignore_index,
+                                  static_cast<int64_t*>(n.data_ptr()), stream_of(labels)),
+           "mt_cross_entropy_count");
+  return n;
+}
+
+at::Tensor ce_sum(const at::Tensor& loss_rows) {
+  const c10::DeviceGuard guard(loss_rows.device());
+  const at::Tensor s = at::empty({}, loss_rows.options());
+  check_rc(mt_cross_entropy_sum(f32_ptr(loss_rows), loss_rows.numel(), f32_ptr(s), stream_of(loss_rows)),
+           "mt_cross_entropy_sum");
+  return s;
+}
+
+std::tuple<at::Tensor, at::Tensor> scale_pair(const at::Tensor& a_in, const at::Tensor& b_in, const at::Tensor& scale) {
+  const c10::DeviceGuard guard(a_in.device());
+  const at::Tensor a = flat(a_in), b = flat(b_in);
+  const at::Tensor s = scale.to(at::kFloat).contiguous();
+  const at::Tensor ao = at::empty(a.sizes(), a.options()), bo = at::empty(b.sizes(), b.options());
+  check_rc(mt_scale_pair(a.data_ptr(), ao.data_ptr(), a.numel(), dtype_code(a), b.data_ptr(), bo.data_ptr(), b.numel(),
+                         dtype_code(b), f32_ptr(s), stream_of(a)),
+           "mt_scale_pair");
+  return {ao, bo};
+}
+
 // --- autograd ----------------------------------------------------------------
 // Forwards run the op below autograd; backwards call the backward ops through
 // the dispatcher.  Gradients that arrive undefined stay undefined except where
@@ -728,6 +757,31 @@ struct RopeFn : torch::autograd::Function<RopeFn> {
   }
 };
 
+// The gradients are computed in the forward and scaled here.
+using CeSig = std::tuple<at::Tensor, at::Tensor, at::Tensor>(const at::Tensor&, const at::Tensor&, const at::Tensor&,
+                                                             int64_t, int64_t, bool);
+struct LinearCeFn : torch::autograd::Function<LinearCeFn> {
+  static variable_list forward(AutogradContext* ctx, const at::Tensor& hidden, const at::Tensor& weight,
+                               const at::Tensor& labels, int64_t ignore_index, int64_t compute, bool need_grad) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    static const auto op = op_handle<CeSig>("mega_trading_amd::fused_linear_ce");
+    auto [loss, gh, gw] = op.call(hidden, weight, labels, ignore_index, compute, need_grad);
+    ctx->save_for_backward({gh, gw});
+    ctx->saved_data["need_grad"] = need_grad;
+    ctx->mark_non_differentiable({gh, gw});
+    ctx->set_materialize_grads(false);
+    return {loss, gh, gw};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    if (!g[0].defined() || !ctx->saved_data["need_grad"].toBool()) return variable_list(6);
+    const auto s = ctx->get_saved_variables();
+    static const auto op = MT_OP(scale_pair);
+    variable_list r(6);
+    std::tie(r[0], r[1]) = op.call(s[0], s[1], g[0]);
+    return r;
+  }
+};
+
 // Whether a call records a gradient: without one the op runs below autograd directly.
 template <class... T>
 bool records(const T&... ts) {
@@ -802,9 +856,22 @@ std::tuple<at::Tensor, at::Tensor> rope_fwd_ad(const at::Tensor& q, const at::Te
   return {r[0], r[1]};
 }
 
+std::tuple<at::Tensor, at::Tensor, at::Tensor> fused_linear_ce_ad(const at::Tensor& hidden, const at::Tensor& weight,
+                                                                  const at::Tensor& labels, int64_t ignore_index,
+                                                                  int64_t compute, bool need_grad) {
+  if (!records(hidden, weight)) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    static const auto op = op_handle<CeSig>("mega_trading_amd::fused_linear_ce");
+    return op.call(hidden, weight, labels, ignore_index, compute, need_grad);
+  }
+  auto r = LinearCeFn::apply(hidden, weight, labels, ignore_index, compute, need_grad);
+  return {r[0], r[1], r[2]};
+}
+
 }  // namespace
 
 TORCH_LIBRARY_IMPL(mega_trading_amd, Autograd, m) {
+  m.impl("fused_linear_ce", &fused_linear_ce_ad);
   m.impl("gqa_attn_fwd", &gqa_attn_fwd_ad);
   m.impl("gqa_rope_attn_fwd", &gqa_rope_attn_fwd_ad);
   m.impl("gqa_rope_attn_packed_fwd", &gqa_rope_attn_packed_fwd_ad);
@@ -842,4 +909,7 @@ TORCH_LIBRARY_IMPL(mega_trading_amd, CUDA, m) {
   m.impl("topk_sample", &topk_sample);
   m.impl("linear_rows", &linear_rows);
   m.impl("linear_rows_gate", &linear_rows_gate);
+  m.impl("ce_count", &ce_count);
+  m.impl("ce_sum", &ce_sum);
+  m.impl("scale_pair", &scale_pair);
 }

@@ -596,6 +596,65 @@ __global__ __launch_bounds__(256) void ce_rows_kernel(void* logits, int64_t ld, 
   }
 }
 
+// The scalars around the rows, one workgroup each (at most kCeScalarRows rows:
+// a CU reads 64 B/clk, 2 us for 32768 labels): *n_valid = the labels that are not
+// ignore_index, and *sum = the rows' losses in a fixed order.
+constexpr int64_t kCeScalarRows = 1 << 17;
+
+__device__ __forceinline__ float block_sum_1024(float v) {
+  __shared__ float part[16];
+  v = wave_reduce<0, false>(v);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  float t = 0.f;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) t += part[w];
+  return t;
+}
+
+__global__ __launch_bounds__(1024) void ce_count_kernel(const int64_t* labels, int64_t rows, int64_t ignore_index,
+                                                        int64_t* n_valid) {
+  float n = 0.f;  // exact: below 2^24
+  for (int64_t i = threadIdx.x; i < rows; i += 1024) n += labels[i] != ignore_index ? 1.f : 0.f;
+  n = block_sum_1024(n);
+  if (threadIdx.x == 0) *n_valid = (int64_t)n;
+}
+
+__global__ __launch_bounds__(1024) void ce_sum_kernel(const float* loss, int64_t rows, float* sum) {
+  float n = 0.f;
+  for (int64_t i = threadIdx.x; i < rows; i += 1024) n += loss[i];
+  n = block_sum_1024(n);
+  if (threadIdx.x == 0) *sum = n;
+}
+
+// The two gradients times the incoming one: out = x * round(*scale), 8 values a
+// thread, the tensor of the first n0 chunks first; the last chunk of each may be
+// short.  One launch instead of two products and two casts of the scalar.
+template <int DT>
+__device__ __forceinline__ void scale_chunk(const void* x, void* out, int64_t n, int64_t c, float s) {
+  s = IO<DT>::round(s);
+  if (8 * c + 8 <= n) {
+    float v[8];
+    IO<DT>::load8(x, 8 * c, v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] *= s;
+    IO<DT>::store8(out, 8 * c, v);
+  } else {
+    for (int64_t i = 8 * c; i < n; ++i) IO<DT>::store1(out, i, IO<DT>::load1(x, i) * s);
+  }
+}
+
+template <int DA, int DB>
+__global__ __launch_bounds__(256) void scale_pair_kernel(const void* a, void* oa, int64_t na, const void* b, void* ob,
+                                                         int64_t nb, const float* scale) {
+  const float s = *scale;
+  const int64_t ca = (na + 7) >> 3, cb = (nb + 7) >> 3;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < ca + cb; i += (int64_t)gridDim.x * 256) {
+    if (i < ca) scale_chunk<DA>(a, oa, na, i, s);
+    else scale_chunk<DB>(b, ob, nb, i - ca, s);
+  }
+}
+
 // ===========================================================================
 // Stand-alone RoPE (triton_ops.py:187-214, kernel :690-761): every
 // interleaved pair (e, o) of q and k becomes (e c - o s, e s + o c), with s

@@ -18,8 +18,8 @@ raise instead (``RuntimeError`` off the GPU or for an unsupported dtype,
 
 Each is a ``torch.library`` op with a fake implementation here and its GPU
 kernels and backward in ``libmt_torch.so`` (``csrc/mt_torch.cpp``), launched on
-the caller's current stream; the loss head, which runs library GEMMs, is a
-Python custom op.
+the caller's current stream; the loss head's forward, which runs library GEMMs,
+is Python.
 """
 
 from __future__ import annotations
@@ -178,8 +178,9 @@ def fused_linear_cross_entropy(
     else:
         compute = torch.promote_types(hidden.dtype, weight.dtype)
     need_grad = torch.is_grad_enabled() and (hidden.requires_grad or weight.requires_grad)
+    _native.ensure()
     with torch.autocast("cuda", enabled=False):
-        loss, _gh, _gw = torch.ops.mega_trading_amd.fused_linear_ce(
+        loss, _gh, _gw = _fused_linear_ce(
             hidden, weight, labels, int(ignore_index), _DT[compute], need_grad)
     return loss
 
@@ -354,13 +355,18 @@ def _topk_sample_fake(logits, noise, k):
 # chunks, and 288 GB of HBM leaves room for the whole logits tensor, so chunking
 # only bounds memory for batches beyond 2 GB of logits.
 _CE_CHUNK_BYTES = 2 << 30
+_CE_SCALAR_ROWS = 1 << 17  # rows of one ce_count / ce_sum launch
+
+# (loss fp32 scalar, d loss / d hidden, d loss / d weight); the gradients are empty tensors when need_grad is False
+_LIB.define("fused_linear_ce(Tensor hidden, Tensor weight, Tensor labels, int ignore_index, int compute_dtype, "
+            "bool need_grad) -> (Tensor, Tensor, Tensor)")
+_LIB.define("ce_count(Tensor labels, int ignore_index) -> Tensor")
+_LIB.define("ce_sum(Tensor loss_rows) -> Tensor")
+_LIB.define("scale_pair(Tensor a, Tensor b, Tensor scale) -> (Tensor, Tensor)")
 
 
-@torch.library.custom_op("mega_trading_amd::fused_linear_ce", mutates_args=(), device_types="cuda")
-def fused_linear_ce(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor, ignore_index: int,
-                    compute_dtype: int, need_grad: bool) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    """(loss fp32 scalar, d loss / d hidden, d loss / d weight); the gradients are
-    empty tensors when need_grad is False."""
+@torch.library.impl(_LIB, "fused_linear_ce", "CUDA")
+def _fused_linear_ce_gpu(hidden, weight, labels, ignore_index, compute_dtype, need_grad):
     lib = _native.load()
     ct = _DTYPE_OF[compute_dtype]
     rows, h = hidden.shape
@@ -374,15 +380,20 @@ def fused_linear_ce(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Te
     if vpad == vocab:
         wc = weight.to(ct).contiguous()
     else:
-        wc = torch.zeros((vpad, h), device=weight.device, dtype=ct)
+        wc = torch.empty((vpad, h), device=weight.device, dtype=ct)
         wc[:vocab].copy_(weight)
+        wc[vocab:].zero_()
     lab = labels.to(torch.int64).contiguous()
-    n_valid = (lab != ignore_index).sum()  # stays on the device: the kernel reads it
+    scalars = 0 < rows <= _CE_SCALAR_ROWS
+    # stays on the device: the kernel reads it
+    n_valid = _ce_count(lab, ignore_index) if scalars else (lab != ignore_index).sum()
     loss_rows = torch.empty((rows,), device=hidden.device, dtype=torch.float32)
+    chunk = max(1, min(rows, _CE_CHUNK_BYTES // (vpad * ct.itemsize)))
+    gw = None
     if need_grad:
         gh = torch.empty((rows, h), device=hidden.device, dtype=ct)
-        gw = torch.zeros((vpad, h), device=hidden.device, dtype=torch.float32)
-    chunk = max(1, min(rows, _CE_CHUNK_BYTES // (vpad * ct.itemsize)))
+        if chunk < rows or not rows:  # several chunks' products are summed in fp32
+            gw = torch.zeros((vpad, h), device=hidden.device, dtype=torch.float32)
     with torch.cuda.device(hidden.device), tuned_gemms():
         stream = _stream(hidden)
         for start in range(0, rows, chunk):
@@ -394,14 +405,15 @@ def fused_linear_ce(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Te
             _native.check(rc, "mt_cross_entropy_rows")
             if need_grad:  # logits now hold d loss / d logits
                 torch.mm(logits, wc, out=gh[start:end])
-                gw.add_(torch.mm(logits.t(), hc[start:end]))
-    loss = loss_rows.sum()
+                part = torch.mm(logits.t(), hc[start:end])
+                gw = part if gw is None else gw.add_(part)
+    loss = _ce_sum(loss_rows) if scalars else loss_rows.sum()
     if not need_grad:
         return loss, hidden.new_empty((0,)), weight.new_empty((0,))
     return loss, gh.to(hidden.dtype), gw[:vocab].to(weight.dtype)
 
 
-@fused_linear_ce.register_fake
+@torch.library.register_fake("mega_trading_amd::fused_linear_ce")
 def _fused_linear_ce_fake(hidden, weight, labels, ignore_index, compute_dtype, need_grad):
     loss = hidden.new_empty((), dtype=torch.float32)
     if not need_grad:
@@ -409,23 +421,10 @@ def _fused_linear_ce_fake(hidden, weight, labels, ignore_index, compute_dtype, n
     return loss, torch.empty_like(hidden), torch.empty_like(weight)
 
 
-def _ce_setup(ctx, inputs, output):
-    _h, _w, _labels, _ignore, _dt, need_grad = inputs
-    _loss, gh, gw = output
-    ctx.need_grad = need_grad
-    ctx.save_for_backward(gh, gw)
-    ctx.mark_non_differentiable(gh, gw)
-    ctx.set_materialize_grads(False)
+@torch.library.register_fake("mega_trading_amd::scale_pair")
+def _scale_pair_fake(a, b, scale):
+    return _like(a), _like(b)
 
-
-def _ce_backward(ctx, dloss, _dgh, _dgw):
-    gh, gw = ctx.saved_tensors
-    if dloss is None or not ctx.need_grad:
-        return None, None, None, None, None, None
-    return gh * dloss.to(gh.dtype), gw * dloss.to(gw.dtype), None, None, None, None
-
-
-fused_linear_ce.register_autograd(_ce_backward, setup_context=_ce_setup)
 
 # the ops as the functions above call them
 _OPS = torch.ops.mega_trading_amd
@@ -437,3 +436,6 @@ _swiglu_fwd = _OPS.swiglu_fwd.default
 _swiglu_packed_fwd = _OPS.swiglu_packed_fwd.default
 _rope_fwd = _OPS.rope_fwd.default
 _topk_sample = _OPS.topk_sample.default
+_fused_linear_ce = _OPS.fused_linear_ce.default
+_ce_count = _OPS.ce_count.default
+_ce_sum = _OPS.ce_sum.default

@@ -11,6 +11,8 @@ rounding step, within 4 ulps), gradients rel 1e-5 in fp32.
 
 from __future__ import annotations
 
+import importlib
+
 import numpy as np
 import pytest
 import torch
@@ -527,3 +529,46 @@ def test_rotary_embedding_hip_route_vs_torch_route(mta):
         torch.testing.assert_close(got.float(), want.float(), rtol=6e-2, atol=6e-2)
     for got, want in ((qa.grad, qb.grad), (ka.grad, kb.grad)):
         torch.testing.assert_close(got.float(), want.float(), rtol=8e-2, atol=8e-2)
+
+
+@pytest.mark.parametrize("rows", [1, 63, 1024, 1025, 131072])
+def test_loss_head_scalars(rows):
+    importlib.import_module("mega-trading_amd._native").ensure()
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    lab = torch.randint(0, 3, (rows,), generator=g, device="cuda")
+    loss = torch.rand(rows, generator=g, device="cuda")
+    o = torch.ops.mega_trading_amd
+    assert int(o.ce_count(lab, 1)) == int((lab != 1).sum())
+    # every addition rounds to 2^-24 of a partial sum: rows / 1024 in a thread, then 6 + 16
+    total = float(loss.double().sum())
+    assert abs(float(o.ce_sum(loss)) - total) <= (rows / 1024 + 23) * 2.0 ** -24 * total
+
+
+@pytest.mark.parametrize("na,nb,da,db", [(8, 8, torch.bfloat16, torch.float32), (13, 7, torch.float16, torch.float16),
+                                         (4099, 1, torch.float32, torch.bfloat16), (0, 24, torch.bfloat16, torch.float32)])
+def test_scale_pair_equals_torch_products(na, nb, da, db):
+    importlib.import_module("mega-trading_amd._native").ensure()
+    a, b = torch.randn(na, device="cuda").to(da), torch.randn(nb, device="cuda").to(db)
+    s = torch.tensor(0.3371, device="cuda")
+    x, y = torch.ops.mega_trading_amd.scale_pair(a, b, s)
+    assert torch.equal(x, a * s.to(da)) and torch.equal(y, b * s.to(db))
+
+
+@pytest.mark.parametrize("rows,dim,dt", [(1, 8, torch.bfloat16), (5, 2056, torch.float32), (4099, 1032, torch.bfloat16),
+                                         (9000, 512, torch.float32), (4097, 4096, torch.float16)])
+def test_add_rms_norm_backward_row_pipeline(rows, dim, dt):
+    """Rows held ahead, the last rows of a grid, and the widest rows (one at a time), against float64."""
+    g = torch.Generator(device="cuda").manual_seed(rows + dim)
+    x, r, dr, dy = (torch.randn(rows, dim, generator=g, device="cuda").to(dt) for _ in range(4))
+    w = (1 + 0.1 * torch.randn(dim, generator=g, device="cuda")).to(dt)
+    args = [t.clone().requires_grad_(True) for t in (x, r, w)]
+    res, y = importlib.import_module("mega-trading_amd.ops").add_rms_norm(*args, eps=1e-5)
+    got = torch.autograd.grad((res, y), args, (dr, dy))
+    s = res.detach().double().requires_grad_(True)
+    wd = w.double().requires_grad_(True)
+    ref_y = s * torch.rsqrt(s.square().mean(-1, keepdim=True) + 1e-5) * wd
+    ds, dw = torch.autograd.grad((s, ref_y), (s, wd), (dr.double(), dy.double()))
+    # one rounding of the result (2^-9, 2^-12) plus fp32 sums; dW also of `rows` products in fp32
+    tol = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -10, torch.float32: 2e-6}[dt]
+    for a, b in ((got[0], ds), (got[1], ds), (got[2], dw)):
+        assert float((a.double() - b).norm() / b.norm()) <= tol
