@@ -181,15 +181,13 @@ void set_pairs(mt::AttnParams& p, int pairs) {
   p.nsb = (p.nqb + p.rb - 1) / p.rb;
 }
 
-// Waves per D = 128 dQ workgroup: 8 (one workgroup per CU) or 4 (two per
-// CU, each barrier then stalls only half of a CU's waves).  Measured at
-// BASELINE config 4 (A/B on one box): 4 waves take the dQ kernel from 0.465
-// to 0.433 ms, but the whole fwd+bwd step stays at 1.51 ms (the dK/dV kernel
-// that follows runs correspondingly slower), so 8 is kept.
-#ifndef MT_DQ128_WAVES
-#define MT_DQ128_WAVES 8
-#endif
-constexpr int kDq128Waves = MT_DQ128_WAVES;
+// Waves per D = 128 dQ workgroup: 4, two workgroups per CU, so that a barrier
+// stalls half of a CU's waves and a small grid spreads over twice the CUs.
+// Against 8 waves (one workgroup per CU), forward + backward: 2 x 500, 32 / 8
+// heads 89.9 -> 80.4 us, 13 x 888, 4 / 4 heads 110.0 -> 107.9, 8 x 2048, 32 / 8
+// heads 1.460 -> 1.452 ms (the dQ kernel gains 7 %, the dK/dV kernel behind it
+// runs at a lower clock).
+constexpr int kDq128Waves = 4;
 
 // Waves per D = 128 forward workgroup: 8 with 128-key K / V tiles (one
 // workgroup per CU, 128 KB of LDS) or 4 with 64-key tiles (two per CU, so a
