@@ -690,6 +690,183 @@ __global__ __launch_bounds__(64 * NW, D <= 64 ? NW / 2 : 2) void attn_fwd_w8_ker
 }
 
 // ===========================================================================
+// Forward for grids that leave CUs idle: keys split over the waves
+// ===========================================================================
+// A workgroup is one (query head, 64-row block): two 32-row waves for each of
+// kSplitGroups key groups.  Every step stages the groups' SUB keys side by side;
+// group g runs fwd32_tile on its own with its own (m, l, O), and the groups are
+// merged through LDS at the end with the log-sum-exp rule.  What bounds a grid of
+// few workgroups is the longest row block's chain of tiles (about 2.5 us per 128
+// keys on a CU of its own), not throughput; this one is a quarter as long, for
+// four times the workgroups and K / V that no other head shares (split_rows in
+// mt_attention.hip: when, and what both take).
+constexpr int kSplitGroups = 4;
+template <int D>
+constexpr int split_keys() { return D <= 64 ? 64 : 32; }  // keys per group and step: 128 KB of LDS at most
+
+template <class E, int D, bool ROPE>
+__global__ __launch_bounds__(128 * kSplitGroups, 2) void attn_fwd_split_kernel(AttnParams p) {
+  using V8 = typename E::v8;
+  using TL = Tile<D>;
+  constexpr int KT = D / 16;
+  constexpr int DT = D / 32;
+  constexpr int S = kSplitGroups, NW = 2 * S, SUB = split_keys<D>();
+  constexpr int TILES = S * SUB / 64;                   // 64-row tiles per step
+  constexpr int SW = TL::INSTR < NW ? TL::INSTR : NW;   // waves that stage tiles
+  constexpr int STAGE = 2 * 2 * TILES * TL::BYTES;      // [buf][K, V][tile]
+  constexpr int MERGE = 2 * (S - 1) * (DT * 4 * 16 + 8) * 64;
+  __shared__ __attribute__((aligned(1024))) char smem[STAGE > MERGE ? STAGE : MERGE];
+  auto kt_lds = [&](int buf) { return smem + buf * 2 * TILES * TL::BYTES; };
+  auto vt_lds = [&](int buf) { return kt_lds(buf) + TILES * TL::BYTES; };
+
+  const int tid = threadIdx.x;
+  const int wave = tid >> 6;
+  const int lane = tid & 63;
+  const int l32 = lane & 31;
+  const int hh = lane >> 5;
+  const int grp = wave >> 1;
+  const int heads = p.B * p.Hq;
+  const int qb = p.nqb - 1 - (int)blockIdx.x / heads;  // longest row blocks first
+  const int head = (int)blockIdx.x % heads % p.Hq;
+  const int b = (int)blockIdx.x % heads / p.Hq;
+  const int kvh = head / p.R;
+  const int q0 = qb * kBlk + 32 * (wave & 1);
+  const bool active = q0 < p.T;
+  const int nstep = (min(p.T, (qb + 1) * kBlk) - 1) / (S * SUB) + 1;
+
+  const uint16_t* kbase = p.k + b * p.sk[0] + (int64_t)kvh * p.sk[1];
+  const uint16_t* vbase = p.v + b * p.sv[0] + (int64_t)kvh * p.sv[1];
+  Stager<D, SW> ks_stage, vs_stage;
+  ks_stage.init(p.sk[2], wave, lane);
+  vs_stage.init(p.sv[2], wave, lane);
+  auto stage = [&](int j, int buf) {
+    if (wave >= SW) return;
+#pragma unroll
+    for (int i = 0; i < TILES; ++i) {
+      const int r0 = (j * TILES + i) * 64;
+      if (r0 >= (qb + 1) * kBlk) break;  // wholly above the row block
+      ks_stage.stage(kt_lds(buf) + i * TL::BYTES, kbase, p.sk[2], r0, p.T);
+      vs_stage.stage(vt_lds(buf) + i * TL::BYTES, vbase, p.sv[2], r0, p.T);
+    }
+  };
+  stage(0, 0);
+
+  // Q^T as B operands, rotated if RoPE (and written out by group 0); rows past
+  // T load row T-1 and are zeroed
+  V8 qop[KT];
+  {
+    const uint16_t* qbase = p.q + b * p.sq[0] + (int64_t)head * p.sq[1];
+    uint16_t* rbase = ROPE ? p.qrot + ((int64_t)b * p.Hq + head) * p.T * D : nullptr;
+    const int row = q0 + l32;
+    const int rc = min(row, p.T - 1);
+    const bool ok = row < p.T;
+    u32x4 x[KT];
+    f32x4 cs[ROPE ? KT : 1], sn[ROPE ? KT : 1];
+#pragma unroll
+    for (int kk = 0; kk < KT; ++kk) {
+      const int d0 = 16 * kk + 8 * hh;
+      x[kk] = *reinterpret_cast<const u32x4*>(qbase + (int64_t)rc * p.sq[2] + d0);
+      if constexpr (ROPE) load_rope_cs<D>(p.cos, p.sin, rc, d0, cs[kk], sn[kk]);
+    }
+#pragma unroll
+    for (int kk = 0; kk < KT; ++kk) {
+      const int d0 = 16 * kk + 8 * hh;
+      u32x4 y = ok ? x[kk] : zero4();
+      if constexpr (ROPE) {
+        y = rope_chunk<E>(y, cs[kk], sn[kk]);
+        if (ok && grp == 0) *reinterpret_cast<u32x4*>(rbase + (int64_t)row * D + d0) = y;
+      }
+      qop[kk] = __builtin_bit_cast(V8, y);
+    }
+  }
+
+  f32x16 oacc[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) zero16(oacc[dt]);
+  float mrun = -INFINITY;
+  float lrun = 0.f;
+  const float c2 = p.scale_log2;
+  const int rbase_op = TL::row_base(lane);
+  const TrBase tbase_op = TL::tr_base(lane);
+  wait_vmem();
+  __syncthreads();
+  for (int j = 0; j < nstep; ++j) {
+    const int buf = j & 1;
+    if (j + 1 < nstep) stage(j + 1, buf ^ 1);
+    const int k0 = (j * S + grp) * SUB;  // the group's first key
+    if (active && k0 <= q0 + 31) {       // wave-uniform
+      const char* K = kt_lds(buf) + grp * SUB * TL::RB;
+      const char* V = vt_lds(buf) + grp * SUB * TL::RB;
+      if (k0 + SUB - 1 <= q0)
+        fwd32_tile<E, D, false, SUB / 32>(K, V, qop, oacc, mrun, lrun, rbase_op, tbase_op, lane, k0, q0, c2);
+      else
+        fwd32_tile<E, D, true, SUB / 32>(K, V, qop, oacc, mrun, lrun, rbase_op, tbase_op, lane, k0, q0, c2);
+    }
+    wait_vmem();
+    __syncthreads();
+  }
+
+  // merge: groups 1 .. S-1 hand (O, m, l) to group 0 of their rows (a group that
+  // had no tile has m = -inf and adds nothing; group 0 always holds key 0)
+  f32x4 (*mo)[DT * 4][64] = reinterpret_cast<f32x4 (*)[DT * 4][64]>(smem);
+  f32x2 (*ml)[64] = reinterpret_cast<f32x2 (*)[64]>(smem + 2 * (S - 1) * DT * 4 * 64 * 16);
+  if (grp > 0) {
+    const int w = wave - 2;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        mo[w][dt * 4 + g][lane] = f32x4{oacc[dt][4 * g], oacc[dt][4 * g + 1], oacc[dt][4 * g + 2], oacc[dt][4 * g + 3]};
+    ml[w][lane] = f32x2{mrun, lrun};
+  }
+  __syncthreads();
+  if (grp > 0) return;
+  float mm = mrun;
+  f32x2 other[S - 1];
+#pragma unroll
+  for (int g = 1; g < S; ++g) {
+    other[g - 1] = ml[2 * (g - 1) + wave][lane];
+    mm = fmaxf(mm, other[g - 1][0]);
+  }
+  const float a0 = exp2_fast(mrun - mm);
+  lrun *= a0;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) oacc[dt][i] *= a0;
+#pragma unroll
+  for (int g = 1; g < S; ++g) {
+    const float a = exp2_fast(other[g - 1][0] - mm);
+    lrun = __builtin_fmaf(a, other[g - 1][1], lrun);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4 o = mo[2 * (g - 1) + wave][dt * 4 + q][lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) oacc[dt][4 * q + e] = __builtin_fmaf(a, o[e], oacc[dt][4 * q + e]);
+      }
+  }
+  mrun = mm;
+  const int row = q0 + l32;
+  if (row >= p.T) return;
+  uint16_t* obase = p.out + b * p.so[0] + (int64_t)head * p.so[1];
+  float* lbase = p.lse + ((int64_t)b * p.Hq + head) * p.T;
+  const float lt = sum_with_partner(lrun);
+  const float inv = 1.f / lt;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int d = dt * 32 + 8 * g + 4 * hh;
+      u32x2 w = {pack2<E>(oacc[dt][4 * g] * inv, oacc[dt][4 * g + 1] * inv),
+                 pack2<E>(oacc[dt][4 * g + 2] * inv, oacc[dt][4 * g + 3] * inv)};
+      *reinterpret_cast<u32x2*>(obase + (int64_t)row * p.so[2] + d) = w;
+    }
+  if (hh == 0) lbase[row] = (mrun + __builtin_amdgcn_logf(lt)) * kLn2;
+}
+
+// ===========================================================================
 // Backward, dQ
 // ===========================================================================
 // One 64-key K/V tile against the wave's 64 query rows: S^T and dP^T

@@ -226,6 +226,21 @@ void copy3(int64_t dst[3], const int64_t* s) {
 #define MT_FWD64_W8 1
 #endif
 
+// Whether a row block's keys are split over the waves of a workgroup of its own
+// (attn_fwd_split_kernel): a quarter of the chain of tiles for four times the
+// workgroups, so it pays while these still fit the CUs, the longer the rows the
+// more of them (two workgroups per CU at D = 32, one above; the D = 128 form's
+// steps are half as wide).  Forward, standard / split, us: D = 64: 1 x 2193, 8
+// heads (280 row blocks) 46.8 / 24.6; 2 x 254, 14 heads (112) 15.2 / 10.9; 2 x
+// 1000, 16 heads (512) 27.6 / 25.1; 8 x 512, 8 heads (512) 19.4 / 21.5; 4 x 1000,
+// 16 heads (1024) 29.1 / 45.8; 1 x 64, 4 heads (4) 8.0 / 9.9.  D = 32: 3 x 1000, 6
+// heads (288) 19.9 / 12.5; 8 x 500, 16 heads (1024) 14.2 / 19.4.  D = 128: 1 x
+// 2000, 4 heads (128) 49.5 / 35.2; 3 x 400, 16 heads (336) 18.9 / 28.9.
+bool split_rows(const mt::AttnParams& p, int D, int cus) {
+  const int64_t blocks = (int64_t)p.B * p.Hq * p.nqb;
+  return p.nqb >= 3 && blocks * (D / 8) <= (int64_t)cus * (p.nqb < 16 ? p.nqb : 16);
+}
+
 template <class E, int D, bool ROPE>
 hipError_t launch_fwd(mt::AttnParams p, hipStream_t st, int) {
   if (ROPE) {
@@ -246,6 +261,9 @@ hipError_t launch_fwd(mt::AttnParams p, hipStream_t st, int) {
   // one resident round (more than one and at most two workgroups per CU):
   // pair heavy and light row blocks on each CU
   const int cus = device_cus();
+  if (split_rows(p, D, cus))
+    return launch_main(mt::attn_fwd_split_kernel<E, D, ROPE>, dim3((unsigned)((int64_t)p.B * p.Hq * p.nqb)),
+                       dim3(128 * mt::kSplitGroups), st, p);
   auto fold = [&](int grid) { return (MT_FWD_FOLD && grid > cus && grid <= 2 * cus) ? cus : 0; };
   const dim3 grid(p.nsb * p.B * p.Hkv * p.n_hsub);
   p.fwd_fold = fold((int)grid.x);

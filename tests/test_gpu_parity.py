@@ -404,3 +404,17 @@ def test_fp32_tile_edges_and_both_forward_forms(b, t, hq, hkv, d, rope):
     for a, r in zip(got, refs):
         err = float((a.double() - r).norm() / max(float(r.norm()), r.numel() ** 0.5))
         assert err <= (t + d) * 2.0 ** -24, err
+
+
+@pytest.mark.parametrize("b,t,hq,hkv,d", [
+    (1, 129, 4, 4, 64), (1, 200, 8, 2, 64), (1, 1025, 7, 1, 64), (2, 257, 14, 2, 64), (1, 511, 3, 1, 32),
+    (2, 1030, 6, 2, 32), (1, 1088, 4, 4, 128), (1, 1217, 6, 2, 128), (1, 128, 2, 1, 64)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_small_grids_split_keys_over_waves(b, t, hq, hkv, d, dt):
+    """Grids small enough for the split-key forward (and dQ): row blocks whose tiles end in every key group,
+    ragged last rows, one call just below the rule (T = 128), fused RoPE; O, LSE and gradients against the oracle."""
+    q, k, v, do = make_inputs(b, t, hq, hkv, d, sigma=1.0, seed=t, dtype=dt)
+    cos, sin = orc.rope_tables(t, d, 10_000.0)
+    pkg = importlib.import_module("mega-trading_amd")
+    compare(run_hip(pkg, q, k, v, do, hq // hkv), oracle(q, k, v, do, hq // hkv))
+    compare(run_hip(pkg, q, k, v, do, hq // hkv, cos, sin), oracle(q, k, v, do, hq // hkv, cos, sin))
