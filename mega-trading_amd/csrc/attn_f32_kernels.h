@@ -87,53 +87,9 @@ __global__ __launch_bounds__(256) void rope_f32_kernel(const float* x, int64_t s
 // LDS tiles of fp32 rows: a row of D floats is laid out, swizzled and copied as
 // a row of 2 D 16-bit values (lds_tile.h).
 // ---------------------------------------------------------------------------
-// Copies of 32 rows by one wave (lds wave-uniform): the offsets of 16 rows, the swizzle's period,
-// are kept and the scalar base moves for the other 16.
+// Copies of 32 rows by one wave (WaveStager, lds_tile.h).
 template <int D>
-struct F32Stager {
-  using TL = Tile<2 * D>;
-  static constexpr int N = TL::NC / 4;      // 1 KB copies of 16 rows
-  static constexpr int COPIES = 2 * N;      // of a tile, whatever path it takes
-  uint32_t voff[N];
-  int lane_;
-
-  static __device__ __forceinline__ void place(int i, int lane, int& row, int& chunk) {
-    const int f = i * 64 + lane;
-    row = f / TL::NC;
-    chunk = (f % TL::NC) ^ TL::swz(row);
-  }
-  __device__ __forceinline__ void init(int64_t row_stride, int lane) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      int row, chunk;
-      place(i, lane, row, chunk);
-      voff[i] = (uint32_t)(row * (int)row_stride + chunk * 4) * 4u;
-    }
-    lane_ = lane;
-  }
-  // rows [row0, row0 + 32) of the matrix at src; rows past T - 1 copy row T - 1
-  __device__ __forceinline__ void stage(char* lds, const float* src, int64_t row_stride, int row0, int T) const {
-    if (row0 + 32 <= T) {
-      const uint32_t l0 = lds_addr(lds);
-#pragma unroll
-      for (int g = 0; g < 2; ++g)
-#pragma unroll
-        for (int i = 0; i < N; ++i)
-          lds_dma16_s(src + (int64_t)(row0 + 16 * g) * row_stride, voff[i], l0 + (g * N + i) * 1024);
-    } else {
-#pragma unroll
-      for (int g = 0; g < 2; ++g)
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          int row, chunk;
-          place(i, lane_, row, chunk);
-          const int grow = min(row0 + 16 * g + row, T - 1);
-          lds_dma16(reinterpret_cast<const uint16_t*>(src + (int64_t)grow * row_stride + chunk * 4),
-                    lds + (g * N + i) * 1024);
-        }
-    }
-  }
-};
+using F32Stager = WaveStager<float, 2 * D, 32>;
 
 // Operand reads of such a tile.
 //  * row: lane (row l32, half hh) reads d values hh D/2 + 4 j .. + 3 (the score
@@ -159,16 +115,6 @@ struct F32Tile {
                                            (tbase ^ (((8 * dt) ^ tr_swz(j)) << 4)));
   }
 };
-
-// All but the wave's newest N copies are done; no LDS read moves across.
-template <int N>
-__device__ __forceinline__ void f32_copies_done() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-// every LDS read a wave has issued is done, before a copy overwrites what they read
-__device__ __forceinline__ void f32_reads_done() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-}
 
 // ---------------------------------------------------------------------------
 // Forward: online softmax over 32-key tiles, O and LSE.  SPLIT = 4: the tiles of
@@ -239,8 +185,8 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_fwd_f32_kernel(Attn
     const bool more = kt + SPLIT <= task.blk;
     // K is here; V may still be on its way (the first time the wave also has its
     // Q loads and Q_rot stores behind the copies)
-    if (kt == kt0) f32_copies_done<0>();
-    else f32_copies_done<F32Stager<D>::COPIES>();
+    if (kt == kt0) copies_done<0>();
+    else copies_done<F32Stager<D>::COPIES>();
     // S^T (lane = query, slots = keys)
     f32x16 s = {};
 #pragma unroll
@@ -249,7 +195,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_fwd_f32_kernel(Attn
 #pragma unroll
       for (int c = 0; c < 4; ++c) s = mfma_f32(k4[c], qv[4 * j + c], s);
     }
-    f32_reads_done();
+    reads_done();
     if (more) kst.stage(K, kbase, p.sk[2], (kt + SPLIT) * 32, p.T);
     if (kt == task.blk) {  // the diagonal; tiles left of it have every key <= every row
 #pragma unroll
@@ -278,13 +224,13 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_fwd_f32_kernel(Attn
 #pragma unroll
       for (int i = 0; i < 16; ++i) oacc[dt][i] *= alpha;
     // O^T += V^T P^T over the tile's 32 keys
-    if (more) f32_copies_done<F32Stager<D>::COPIES>();
-    else f32_copies_done<0>();
+    if (more) copies_done<F32Stager<D>::COPIES>();
+    else copies_done<0>();
 #pragma unroll
     for (int j = 0; j < 16; ++j)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) oacc[dt] = mfma_f32(tile.tr(V, j, dt), s[j], oacc[dt]);
-    f32_reads_done();
+    reads_done();
     if (more) vst.stage(V, vbase, p.sv[2], (kt + SPLIT) * 32, p.T);
   }
   if constexpr (SPLIT == 4) {
@@ -438,8 +384,8 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_bwd_dq_f32_kernel(A
   // dP first, then S: V's next tile is copied behind S and dQ, K's behind the next dP
   for (int kt = kt0; kt <= task.blk; kt += SPLIT) {
     const bool more = kt + SPLIT <= task.blk;
-    if (kt == kt0) f32_copies_done<0>();
-    else f32_copies_done<F32Stager<D>::COPIES>();
+    if (kt == kt0) copies_done<0>();
+    else copies_done<F32Stager<D>::COPIES>();
     f32x16 s = {}, dp = {};
 #pragma unroll
     for (int j = 0; j < HD / 4; ++j) {
@@ -447,12 +393,12 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_bwd_dq_f32_kernel(A
 #pragma unroll
       for (int c = 0; c < 4; ++c) dp = mfma_f32(v4[c], gv[4 * j + c], dp);
     }
-    f32_reads_done();
+    reads_done();
     if (more) {
       vst.stage(V, vbase, p.sv[2], (kt + SPLIT) * 32, p.T);
-      f32_copies_done<F32Stager<D>::COPIES>();
+      copies_done<F32Stager<D>::COPIES>();
     } else {
-      f32_copies_done<0>();
+      copies_done<0>();
     }
 #pragma unroll
     for (int j = 0; j < HD / 4; ++j) {
@@ -473,7 +419,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_bwd_dq_f32_kernel(A
     for (int j = 0; j < 16; ++j)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) dq[dt] = mfma_f32(tile.tr(K, j, dt), s[j], dq[dt]);
-    f32_reads_done();
+    reads_done();
     if (more) kst.stage(K, kbase, p.sk[2], (kt + SPLIT) * 32, p.T);
   }
   if constexpr (SPLIT == 4) {
@@ -594,7 +540,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_bwd_dkv_f32_kernel(
     const bool more = u + 4 < npair;
     // S and dP: rows m = the tile's queries, lane = key
     f32x16 s = {}, dp = {};
-    f32_copies_done<F32Stager<D>::COPIES + 1>();  // Q (dO and its vectors may still be on their way)
+    copies_done<F32Stager<D>::COPIES + 1>();  // Q (dO and its vectors may still be on their way)
 #pragma unroll
     for (int j = 0; j < HD / 4; ++j) {
       const f32x4 q4 = tile.row(Qt, j);
@@ -604,7 +550,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_bwd_dkv_f32_kernel(
         if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // a few operands in flight, not all
       }
     }
-    f32_copies_done<0>();
+    copies_done<0>();
 #pragma unroll
     for (int j = 0; j < HD / 4; ++j) {
       const f32x4 g4 = tile.row(Gt, j);
@@ -642,7 +588,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_bwd_dkv_f32_kernel(
         if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
       }
     }
-    f32_reads_done();
+    reads_done();
     if (more) stage_q(u + 4);
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
@@ -652,7 +598,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_bwd_dkv_f32_kernel(
         if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
       }
     }
-    f32_reads_done();
+    reads_done();
     if (more) stage_g(u + 4);
   }
   __syncthreads();  // every wave's tiles are read: the block is reused for the sums

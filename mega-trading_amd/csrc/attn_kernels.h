@@ -1118,6 +1118,160 @@ __device__ __forceinline__ void dq_body(const AttnParams& p, int L, char* lds) {
 
 
 // ===========================================================================
+// Backward, dQ for grids that leave CUs idle (D <= 64): keys split over waves
+// ===========================================================================
+// The task of a workgroup is one (query head, 64-row block); wave w takes the
+// 64-key tiles w, w + 4, ... through dq_tile, each copied into LDS of its own
+// with no barrier, and the four partial sums are added through LDS.  As in
+// attn_fwd_split_kernel, a quarter of the longest chain of tiles for four times
+// the workgroups.  One tile buffer per wave keeps two workgroups on a CU; the
+// co-resident one hides the copies.
+template <int D>
+struct DqSplitLds {
+  static constexpr int WAVE = 2 * Tile<D>::BYTES;  // a wave's K and V tile
+  static constexpr int RED = (2 * (D / 32)) * 3 * 4 * 64 * 16;
+  static constexpr int TILES = 4 * WAVE > RED ? 4 * WAVE : RED;
+  static constexpr int BYTES = TILES + kDqOffsFloats * 4;  // then the row block's offsets
+};
+
+template <class E, int D, bool ROPE>
+__device__ __forceinline__ void dq_split_body(const AttnParams& p, int L, char* lds) {
+  static_assert(D <= 64, "register budget");
+  using V8 = typename E::v8;
+  using TL = Tile<D>;
+  constexpr int KT = D / 16;
+  constexpr int DT = D / 32;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int l32 = lane & 31;
+  const int hh = lane >> 5;
+  const int heads = p.B * p.Hq;
+  const int qb = p.nqb - 1 - L / heads;  // longest row blocks first
+  const int head = L % heads % p.Hq;
+  const int b = L % heads / p.Hq;
+  const int kvh = head / p.R;
+  const int q0 = qb * kBlk;
+  float* offs = reinterpret_cast<float*>(lds + DqSplitLds<D>::TILES);
+  char* K = lds + wave * DqSplitLds<D>::WAVE;
+  char* V = K + TL::BYTES;
+
+  const uint16_t* kbase = p.k + b * p.sk[0] + (int64_t)kvh * p.sk[1];
+  const uint16_t* vbase = p.v + b * p.sv[0] + (int64_t)kvh * p.sv[1];
+  const int64_t rowbase = ((int64_t)b * p.Hq + head) * p.T;
+  WaveStager<uint16_t, D, 64> kst, vst;
+  kst.init(p.sk[2], lane);
+  vst.init(p.sv[2], lane);
+  if (wave <= qb) {
+    kst.stage(K, kbase, p.sk[2], wave * kBlk, p.T);
+    vst.stage(V, vbase, p.sv[2], wave * kBlk, p.T);
+  }
+
+  V8 qop[2][KT], gop[2][KT];
+  {
+    const uint16_t* qbase = p.q + b * p.sq[0] + (int64_t)head * p.sq[1];
+    const uint16_t* gbase = p.dout + b * p.sdo[0] + (int64_t)head * p.sdo[1];
+    u32x4 qx[2][KT], gx[2][KT];
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      const int rc = min(q0 + nt * 32 + l32, p.T - 1);
+#pragma unroll
+      for (int kk = 0; kk < KT; ++kk) {
+        const int d0 = 16 * kk + 8 * hh;
+        qx[nt][kk] = *reinterpret_cast<const u32x4*>(qbase + (int64_t)rc * p.sq[2] + d0);
+        gx[nt][kk] = *reinterpret_cast<const u32x4*>(gbase + (int64_t)rc * p.sdo[2] + d0);
+      }
+    }
+    // the row block's offsets (dq_offset_tile), shared: waves 0 / 1 fill rows 0-31 / 32-63
+    if (wave < 2) {
+      const int row = q0 + wave * 32 + l32;
+      const float nlse2 = row < p.T ? p.nlse2[rowbase + row] : 0.f;
+      const float ndelta = row < p.T ? p.ndelta[rowbase + row] : 0.f;
+      const f32x4 nl = {nlse2, nlse2, nlse2, nlse2}, nd = {ndelta, ndelta, ndelta, ndelta};
+#pragma unroll
+      for (int g = 2 * hh; g < 2 * hh + 2; ++g) {
+        *reinterpret_cast<f32x4*>(offs + (0 * 2 + wave) * 512 + g * 128 + l32 * 4) = nl;
+        *reinterpret_cast<f32x4*>(offs + (1 * 2 + wave) * 512 + g * 128 + l32 * 4) = nd;
+      }
+    }
+    const float c2 = p.scale_log2;
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      const bool ok = q0 + nt * 32 + l32 < p.T;
+#pragma unroll
+      for (int kk = 0; kk < KT; ++kk) {
+        u32x4 qs = ok ? qx[nt][kk] : zero4();  // pre-multiplied by scale * log2(e), as in dq_body
+#pragma unroll
+        for (int w = 0; w < 4; ++w) qs[w] = pack2<E>(lo_f<E>(qs[w]) * c2, hi_f<E>(qs[w]) * c2);
+        qop[nt][kk] = __builtin_bit_cast(V8, qs);
+        gop[nt][kk] = __builtin_bit_cast(V8, ok ? gx[nt][kk] : zero4());
+      }
+    }
+  }
+  f32x16 dqacc[DT][2];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) zero16(dqacc[dt][nt]);
+  const int rbase_op = TL::row_base(lane);
+  const TrBase tbase_op = TL::tr_base(lane);
+  __syncthreads();  // the offsets
+  int j = wave;
+  for (; j < qb; j += 4) {
+    copies_done<0>();
+    dq_tile<E, D, false>(K, V, qop, gop, dqacc, offs, rbase_op, tbase_op, l32, hh);
+    reads_done();
+    if (j + 4 <= qb) {
+      kst.stage(K, kbase, p.sk[2], (j + 4) * kBlk, p.T);
+      vst.stage(V, vbase, p.sv[2], (j + 4) * kBlk, p.T);
+    }
+  }
+  if (j == qb) {  // the diagonal tile
+    copies_done<0>();
+    dq_tile<E, D, true>(K, V, qop, gop, dqacc, offs, rbase_op, tbase_op, l32, hh);
+  }
+  __syncthreads();  // every wave's tiles are read: the block is reused for the sums
+
+  // piece (nt, dt) of the row block is finished by one wave, from the other three's sums
+  f32x4 (*red)[3][4][64] = reinterpret_cast<f32x4 (*)[3][4][64]>(lds);
+#pragma unroll
+  for (int pc = 0; pc < 2 * DT; ++pc) {
+    if (wave == pc) continue;
+    const f32x16& a = dqacc[pc % DT][pc / DT];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      red[pc][wave - (wave > pc ? 1 : 0)][g][lane] = f32x4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+  }
+  __syncthreads();
+  uint16_t* dqbase = p.out + b * p.sout[0] + (int64_t)head * p.sout[1];
+#pragma unroll
+  for (int pc = 0; pc < 2 * DT; ++pc) {
+    if (wave != pc) continue;
+    const int nt = pc / DT, dt = pc % DT;
+    f32x16& a = dqacc[dt][nt];
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 o = red[pc][s][g][lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[4 * g + e] += o[e];
+      }
+    const int row = q0 + nt * 32 + l32;
+    if (row >= p.T) continue;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int d = dt * 32 + 8 * g + 4 * hh;
+      float x0 = a[4 * g] * p.scale, x1 = a[4 * g + 1] * p.scale;
+      float x2 = a[4 * g + 2] * p.scale, x3 = a[4 * g + 3] * p.scale;
+      if constexpr (ROPE)
+        rope_back4(x0, x1, x2, x3, p.cos + (int64_t)row * (D / 2) + d / 2, p.sin + (int64_t)row * (D / 2) + d / 2);
+      u32x2 w = {pack2<E>(x0, x1), pack2<E>(x2, x3)};
+      *reinterpret_cast<u32x2*>(dqbase + (int64_t)row * p.sout[2] + d) = w;
+    }
+  }
+}
+
+// ===========================================================================
 // Backward, dQ for D = 128: 8 waves of 32 query rows per workgroup
 // ===========================================================================
 // As for the D = 128 forward: the 4 (head, 64-row block) pairs of a RowTask
@@ -1736,15 +1890,13 @@ __global__ __launch_bounds__(64 * kKvWaves, D <= 64 ? 2 : 1) void attn_bwd_dkv_k
 // tasks of a group share one XCD's L2 (its K/V and Q/dO rows).  When a count
 // is not a multiple of 8 the merge is per workgroup.  KVK = keys per dK/dV
 // task (dkv_body).
-template <int D>
-struct BwdLds {
-  static constexpr int BYTES = DqLds<D>::BYTES > DkvLds<D>::BYTES ? DqLds<D>::BYTES : DkvLds<D>::BYTES;
-};
-
-template <class E, int D, bool ROPE, bool PEEL, int KVK>
+// DQ: the form of the dQ tasks -- 0 / 1: dq_body without / with PEEL, kDqSplit: dq_split_body.
+constexpr int kDqSplit = 2;
+template <class E, int D, bool ROPE, int DQ, int KVK>
 __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(AttnParams p) {
   static_assert(kKvWaves == 4, "dQ and dK/dV workgroups must have the same size");
-  __shared__ __attribute__((aligned(1024))) char lds[BwdLds<D>::BYTES];
+  constexpr int DQ_LDS = DQ == kDqSplit ? DqSplitLds<D>::BYTES : DqLds<D>::BYTES;
+  __shared__ __attribute__((aligned(1024))) char lds[DQ_LDS > DkvLds<D>::BYTES ? DQ_LDS : DkvLds<D>::BYTES];
   const int L = blockIdx.x;
   const int sh = ((p.n_kv_tasks | p.n_dq_tasks) & 7) == 0 ? 3 : 0;  // chunks of 8 workgroups, or of 1
   const int n = (p.n_kv_tasks + p.n_dq_tasks) >> sh;
@@ -1780,8 +1932,10 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_kernel(AttnParams p) {
   }
   if (kv)
     dkv_body<E, D, ROPE, KVK, true>(p, (idx << sh) + sub, lds);
+  else if constexpr (DQ == kDqSplit)
+    dq_split_body<E, D, ROPE>(p, (idx << sh) + sub, lds);
   else
-    dq_body<E, D, ROPE, PEEL>(p, (idx << sh) + sub, lds);
+    dq_body<E, D, ROPE, DQ != 0>(p, (idx << sh) + sub, lds);
 }
 
 // ===========================================================================

@@ -197,6 +197,68 @@ struct Stager {
   }
 };
 
+// Copies of ROWS rows by one wave into LDS of its own (lds wave-uniform), W the
+// row width in 16-bit values, T the element type of the matrix: the offsets of
+// 16 rows, the swizzle's period, are kept and the scalar base moves for the
+// others.  The wave waits for them by count (copies_done), with no barrier.
+template <class T, int W, int ROWS>
+struct WaveStager {
+  using TL = Tile<W>;
+  static constexpr int G = ROWS / 16;
+  static constexpr int N = TL::NC / 4;       // 1 KB copies of 16 rows
+  static constexpr int COPIES = G * N;       // of a tile, whatever path it takes
+  static constexpr int EL = 16 / sizeof(T);  // elements per 16-byte chunk
+  uint32_t voff[N];
+  int lane_;
+
+  static __device__ __forceinline__ void place(int i, int lane, int& row, int& chunk) {
+    const int f = i * 64 + lane;
+    row = f / TL::NC;
+    chunk = (f % TL::NC) ^ TL::swz(row);
+  }
+  __device__ __forceinline__ void init(int64_t row_stride, int lane) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      int row, chunk;
+      place(i, lane, row, chunk);
+      voff[i] = (uint32_t)(row * (int)row_stride + chunk * EL) * (uint32_t)sizeof(T);
+    }
+    lane_ = lane;
+  }
+  // rows [row0, row0 + ROWS) of the matrix at src; rows past T_ - 1 copy row T_ - 1
+  __device__ __forceinline__ void stage(char* lds, const T* src, int64_t row_stride, int row0, int T_) const {
+    if (row0 + ROWS <= T_) {
+      const uint32_t l0 = lds_addr(lds);
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+          lds_dma16_s(src + (int64_t)(row0 + 16 * g) * row_stride, voff[i], l0 + (g * N + i) * 1024);
+    } else {
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          int row, chunk;
+          place(i, lane_, row, chunk);
+          const int grow = min(row0 + 16 * g + row, T_ - 1);
+          lds_dma16(reinterpret_cast<const uint16_t*>(src + (int64_t)grow * row_stride + chunk * EL),
+                    lds + (g * N + i) * 1024);
+        }
+    }
+  }
+};
+
+// All but the wave's newest N copies are done; no LDS read moves across.
+template <int N>
+__device__ __forceinline__ void copies_done() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// every LDS read a wave has issued is done, before a copy overwrites what they read
+__device__ __forceinline__ void reads_done() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
+
 // Stage 64 fp32 values (row-indexed vector, clamped at T-1) with one wave.
 __device__ __forceinline__ void stage_vec64(char* lds, const float* src, int row0, int T, int lane) {
   if (row0 + 64 <= T)

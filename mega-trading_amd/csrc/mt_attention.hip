@@ -321,7 +321,7 @@ int merged_dkv_keys(const mt::AttnParams& p) {
 // task of the other.  Measured at BASELINE config 3 against a proportional
 // interleave of the whole lists (which starts the medium dK/dV tasks last):
 // see the design notes; the end of the launch is its shortest tasks.
-void bwd_merge(mt::AttnParams& p, int kvk) {
+void bwd_merge(mt::AttnParams& p, int kvk, bool dq_split) {
   const int sh = ((p.n_kv_tasks | p.n_dq_tasks) & 7) == 0 ? 3 : 0;
   const int nk = p.n_kv_tasks >> sh, nd = p.n_dq_tasks >> sh;
   p.mg_mid_kv = p.mg_mid_dq = 0;
@@ -331,12 +331,13 @@ void bwd_merge(mt::AttnParams& p, int kvk) {
     return;
   }
   const long hpt = (p.R + p.n_split - 1) / p.n_split;
-  const int kv_groups = p.B * p.Hkv * p.n_split, dq_groups = p.B * p.Hkv * p.n_hsub;
+  const int kv_groups = p.B * p.Hkv * p.n_split, dq_groups = dq_split ? p.B * p.Hq : p.B * p.Hkv * p.n_hsub;
   auto wk = [&](int q) {
     const int kb = (q << sh) / kv_groups;
     return (kvk == 128 ? 64L : 32L) * hpt * ((p.T - kvk * kb + 127) / 128);
   };
   auto wd = [&](int r) {
+    if (dq_split) return 48L * ((p.nqb - 1 - (r << sh) / dq_groups) / 4 + 1);
     const int sb = p.nsb - 1 - (r << sh) / dq_groups;
     return 48L * std::min((sb + 1) * p.rb, p.nqb);
   };
@@ -354,11 +355,25 @@ void bwd_merge(mt::AttnParams& p, int kvk) {
   p.mg_mid_dq = std::max(0, nd - head_d - tail_d);
 }
 
+// Whether the one-launch backward's dQ tasks split their keys over the waves
+// (dq_split_body), as split_rows for the forward: while one (head, 64-row block)
+// a workgroup fits two resident workgroups per CU, twice that for long rows of D =
+// 32.  Forward + backward, standard / split, us: D = 64: 1 x 2193, 8 heads (280 row
+// blocks) 90.3 / 65.9; 1 x 4000, 4 heads (252) 137 / 92; 2 x 254, 14 heads (112)
+// 36.4 / 28.3; 2 x 1000, 16 heads (512) 67.8 / 62.8; 2 x 600, 32 heads (640) 57.9 /
+// 62.6; 4 x 1000, 16 heads (1024) 88.0 / 90.3.  D = 32: 6 x 1000, 12 heads (1152)
+// 72.6 / 66.7; 8 x 500, 16 heads (1024) 41.8 / 44.0.
+bool split_dq(const mt::AttnParams& p, int D) {
+  const int64_t blocks = (int64_t)p.B * p.Hq * p.nqb;
+  return p.nqb >= 3 && blocks <= (D <= 32 && p.nqb >= 16 ? 4 : 2) * (int64_t)device_cus();
+}
+
 // stage: 1 = prep (delta, LSE log2 e) + dQ, 2 = dK/dV (reads the prep vectors), 3 = all
 template <class E, int D, bool ROPE>
 hipError_t launch_bwd(mt::AttnParams p, hipStream_t st, int stage) {
-  const int n_dq = p.nsb * p.B * p.Hkv * p.n_hsub;
   const int kvk = D <= 64 ? merged_dkv_keys(p) : mt::kKvKeys;
+  const bool dq_split = D <= 64 && kvk == 64 && split_dq(p, D);
+  const int n_dq = dq_split ? p.B * p.Hq * p.nqb : p.nsb * p.B * p.Hkv * p.n_hsub;
   const int n_kv = (p.T + kvk - 1) / kvk * p.B * p.Hkv * p.n_split;
   if (D <= 64 && (stage & 1)) {
     // -delta and -LSE log2(e) for both kinds of task (at D = 128 the dQ
@@ -374,15 +389,17 @@ hipError_t launch_bwd(mt::AttnParams p, hipStream_t st, int stage) {
     // dQ and dK/dV tasks in one grid
     p.n_dq_tasks = (stage & 1) ? n_dq : 0;
     p.n_kv_tasks = (stage & 2) ? n_kv : 0;
-    bwd_merge(p, kvk);
+    bwd_merge(p, kvk, dq_split);
     const dim3 grid(p.n_dq_tasks + p.n_kv_tasks);
     hipError_t e;
-    if (kvk == 64)
-      e = p.rb == 1 ? launch_main(mt::attn_bwd_kernel<E, D, ROPE, true, 64>, grid, dim3(256), st, p)
-                    : launch_main(mt::attn_bwd_kernel<E, D, ROPE, false, 64>, grid, dim3(256), st, p);
+    if (dq_split)
+      e = launch_main(mt::attn_bwd_kernel<E, D, ROPE, mt::kDqSplit, 64>, grid, dim3(256), st, p);
+    else if (kvk == 64)
+      e = p.rb == 1 ? launch_main(mt::attn_bwd_kernel<E, D, ROPE, 1, 64>, grid, dim3(256), st, p)
+                    : launch_main(mt::attn_bwd_kernel<E, D, ROPE, 0, 64>, grid, dim3(256), st, p);
     else
-      e = p.rb == 1 ? launch_main(mt::attn_bwd_kernel<E, D, ROPE, true, 128>, grid, dim3(256), st, p)
-                    : launch_main(mt::attn_bwd_kernel<E, D, ROPE, false, 128>, grid, dim3(256), st, p);
+      e = p.rb == 1 ? launch_main(mt::attn_bwd_kernel<E, D, ROPE, 1, 128>, grid, dim3(256), st, p)
+                    : launch_main(mt::attn_bwd_kernel<E, D, ROPE, 0, 128>, grid, dim3(256), st, p);
     if (e != hipSuccess) return e;
   } else {
     if (stage & 1) {

@@ -115,15 +115,16 @@ def test_the_checks_catch_the_hazards():
     assert _wait_states(["s_nop 4"]) == 5 and _wait_states(["v_mov_b32 v1, 0", "s_nop 2"]) == 4
 
 
-def test_fp32_kernels_copies_have_their_wait_states(tmp_path):
-    """The fp32 kernels' wave-private copies: the same rules, and M0 written by scalar instructions only."""
+def test_wave_private_and_split_copies_have_their_wait_states(tmp_path):
+    """The fp32 and the split-key kernels' copies: the same rules, and M0 written by scalar instructions only."""
     hipcc = _hipcc()
     if hipcc is None:
         pytest.skip("hipcc not available")
     src, out = tmp_path / "tu.hip", tmp_path / "tu.s"
     src.write_text('#include "attn_f32_kernels.h"\n' + "".join(
         f"template __global__ void mt::{k}(mt::AttnParams);\n"
-        for k in ("attn_fwd_f32_kernel<32, true, 4>", "attn_fwd_f32_kernel<64, false, 1>",
+        for k in ("attn_bwd_kernel<mt::BF16, 64, false, mt::kDqSplit, 64>", "attn_fwd_split_kernel<mt::FP16, 32, true>",
+                  "attn_fwd_split_kernel<mt::BF16, 128, false>", "attn_fwd_f32_kernel<32, true, 4>", "attn_fwd_f32_kernel<64, false, 1>",
                   "attn_bwd_dq_f32_kernel<128, true, 1>", "attn_bwd_dkv_f32_kernel<64, true>")))
     proc = subprocess.run([hipcc, "--offload-arch=gfx950", "-O3", "-std=c++17", "--cuda-device-only", "-S",
                            "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-pass-failed",
