@@ -531,7 +531,7 @@ def test_rotary_embedding_hip_route_vs_torch_route(mta):
         torch.testing.assert_close(got.float(), want.float(), rtol=8e-2, atol=8e-2)
 
 
-@pytest.mark.parametrize("rows", [1, 63, 1024, 1025, 131072])
+@pytest.mark.parametrize("rows", [1, 63, 1024, 1025, 16383, 16385, 131072])
 def test_loss_head_scalars(rows):
     importlib.import_module("mega-trading_amd._native").ensure()
     g = torch.Generator(device="cuda").manual_seed(rows)
