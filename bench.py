@@ -331,13 +331,12 @@ def time_decode(pkg, cases=DECODE_CASES, iters=50):
     (32 rollouts, Hq 8, Hkv 2, D 64, bf16 cache of `capacity` positions:
     1024 = the config's block_size, and 512 for a shorter window), through the
     C ABI with preallocated buffers, the length read from device memory as the
-    recorded decode step does: the attention (mt_gqa_attn_decode_dev: the
-    split + combine pair for a 1024-position cache, the fused one-launch
-    kernel for at most 512) and the RoPE / cache-append kernel, each timed
+    recorded decode step does: the attention (mt_gqa_attn_decode_dev: one
+    launch at these capacities) and the RoPE / cache-append kernel, each timed
     over `iters` back-to-back launches with HIP events.  Algorithmic bytes:
     the attention reads the group's q and L cached K and V rows once and
-    writes O; the split + combine pair also writes and reads one fp32 partial
-    (o, m, l) per head and 64-key split; the append reads the fp32 q / k / v
+    writes O; a longer cache also writes and reads one fp32 partial
+    (o, m, l) per head and 256 keys; the append reads the fp32 q / k / v
     projections and writes q_rot and one K and one V cache row."""
     native = pkg._native
     lib = native.load()
@@ -377,7 +376,8 @@ def time_decode(pkg, cases=DECODE_CASES, iters=50):
         q_rot = torch.empty_like(q)
         ins = (ctypes.c_int64 * 6)(xq.stride(0), xq.stride(1), xk.stride(0), xk.stride(1), xv.stride(0), xv.stride(1))
         cst = (ctypes.c_int64 * 6)(*kc.stride()[:3], *vc.stride()[:3])
-        fused = (cap + 63) // 64 <= 8  # the library's rule: at most 8 splits of 64 keys in one launch
+        # the library's rule: one launch up to 512 keys, up to 1024 at D <= 64 with 64 (sequence, KV head) pairs
+        fused = cap <= 512 or (cap <= 1024 and d <= 64 and b * hkv >= 64)
         ns = (L + 63) // 64
         attn = lambda: native.check(lib.mt_gqa_attn_decode_dev(  # noqa: E731
             q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), b, hq, hkv, cap, length.data_ptr(), d, st,

@@ -194,7 +194,7 @@ int mt_time_kernel_queue(void* const* start_events, void* const* stop_events, in
  *   (rotated keys), o [B,Hq,1,D] written; strides: 16 int64 = q, k_cache,
  *   v_cache, o in (b, h, t, d) order (the t stride of q and o is unused).
  *   Hq / Hkv <= 8; L >= 1.  The fp32 workspace (16-byte aligned) holds one
- *   partial per 64-key split (mt_gqa_attn_decode_workspace_size).
+ *   partial per 256 keys (mt_gqa_attn_decode_workspace_size).
  */
 size_t mt_gqa_attn_decode_workspace_size(int B, int Hq, int L, int D);
 int mt_gqa_attn_decode(const void* q, const void* k_cache, const void* v_cache, void* o, int B, int Hq, int Hkv,
