@@ -378,7 +378,7 @@ def time_decode(pkg, cases=DECODE_CASES, iters=50):
         cst = (ctypes.c_int64 * 6)(*kc.stride()[:3], *vc.stride()[:3])
         # the library's rule: one launch up to 512 keys, up to 1024 at D <= 64 with 64 (sequence, KV head) pairs
         fused = cap <= 512 or (cap <= 1024 and d <= 64 and b * hkv >= 64)
-        ns = (L + 63) // 64
+        ns = (L + 255) // 256
         attn = lambda: native.check(lib.mt_gqa_attn_decode_dev(  # noqa: E731
             q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), b, hq, hkv, cap, length.data_ptr(), d, st,
             scale, native.DTYPE_BF16, ws.data_ptr(), ws_bytes, sp), "mt_gqa_attn_decode_dev")
@@ -388,7 +388,7 @@ def time_decode(pkg, cases=DECODE_CASES, iters=50):
             native.DTYPE_BF16, sp), "mt_decode_rope_append")
         attn_bytes = 2 * b * hkv * L * d * 2 + 2 * b * hq * d * 2
         if not fused:
-            attn_bytes += 2 * b * hq * ns * (d + 2) * 4
+            attn_bytes += 2 * b * hq * ns * (d + 4) * 4
         us = timed(attn, iters)
         us_app = timed(append, iters)
         app_bytes = b * (hq + 2 * hkv) * d * 4 + b * (hq + 2 * hkv) * d * 2 + d * 4
