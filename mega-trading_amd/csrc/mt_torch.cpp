@@ -17,9 +17,12 @@
 // place under the same rule.  Errors from the C ABI are raised as RuntimeError with
 // mt_last_error()'s message.
 #include <ATen/ATen.h>
+#include <ATen/FuncTorchTLS.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <torch/library.h>
 
 #include <array>
@@ -537,7 +540,7 @@ std::tuple<at::Tensor, at::Tensor> scale_pair(const at::Tensor& a_in, const at::
 // --- autograd ----------------------------------------------------------------
 // Forwards run the op below autograd; backwards call the backward ops through
 // the dispatcher.  Gradients that arrive undefined stay undefined except where
-// noted.  As before, none of these has a double backward or a forward-mode rule.
+// noted.  A forward-mode tangent on a recorded call is refused.
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 using Opt = std::optional<at::Tensor>;
@@ -868,9 +871,52 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> fused_linear_ce_ad(const at::Tens
   return {r[0], r[1], r[2]};
 }
 
+// An op without a formula (the backward ops among them: no double backward)
+// refuses a gradient instead of dropping it: its outputs' node raises.  torch's
+// own fallback for such ops only warns and passes no gradient on.  Caches that an
+// op writes keep their own autograd state.
+void no_formula(const c10::OperatorHandle& op, c10::DispatchKeySet ks, torch::jit::Stack* stack) {
+  variable_list recorded;
+  bool tangent = false;
+  if (c10::GradMode::is_enabled()) {
+    auto look = [&](const at::Tensor& t) {
+      if (!t.defined()) return;
+      if (t.requires_grad()) recorded.push_back(t);
+      tangent |= t._fw_grad(0).defined();
+    };
+    for (const c10::IValue& a : torch::jit::last(*stack, op.schema().arguments().size())) {
+      if (a.isTensor()) look(a.toTensor());
+      else if (a.isTensorList())
+        for (const at::Tensor& t : a.toTensorList()) look(t);
+    }
+  }
+  if (!recorded.empty()) {
+    if (const auto& f = at::functorch::functorchTLSAccessor()) f->checkSupportsCppAutogradFunction();
+    TORCH_CHECK(!tangent, op.schema().name(), " has no forward-mode derivative");
+  }
+  {
+    at::AutoDispatchBelowAutograd below;
+    op.redispatchBoxed(ks & c10::after_autograd_keyset, stack);
+  }
+  if (recorded.empty()) return;
+  const std::shared_ptr<torch::autograd::Node> node(
+      new torch::autograd::Error(
+          "Trying to backward through " + op.schema().name() + " but no autograd formula was registered",
+          torch::autograd::collect_next_edges(recorded)),
+      torch::autograd::deleteNode);
+  for (const c10::IValue& r : torch::jit::last(*stack, op.schema().returns().size()))
+    if (r.isTensor() && torch::autograd::isDifferentiableType(r.toTensor().scalar_type()))
+      torch::autograd::set_history(r.toTensor(), node);
+}
+
 }  // namespace
 
 TORCH_LIBRARY_IMPL(mega_trading_amd, Autograd, m) {
+  // gqa_attn_bwd_packed keeps torch's fallback, a warning, which it has always had
+  for (const char* op : {"gqa_attn_bwd", "gqa_attn_decode", "gqa_attn_decode_dev", "decode_rope_append",
+                         "gqa_attn_decode_append", "rms_norm_bwd", "add_rms_norm_bwd", "rms_norm_bwd_mixed", "swiglu_bwd",
+                         "swiglu_packed_bwd", "topk_sample", "linear_rows", "linear_rows_gate", "ce_sum", "scale_pair"})
+    m.impl(op, torch::CppFunction::makeFromBoxedFunction<&no_formula>());
   m.impl("fused_linear_ce", &fused_linear_ce_ad);
   m.impl("gqa_attn_fwd", &gqa_attn_fwd_ad);
   m.impl("gqa_rope_attn_fwd", &gqa_rope_attn_fwd_ad);

@@ -1,0 +1,102 @@
+"""CPU tests of the ops' autograd rules, on meta tensors (shapes only, nothing is launched).
+
+What has no formula must refuse a gradient: dropping it gives a caller wrong
+gradients without an error.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+BF16 = torch.bfloat16
+
+
+@pytest.fixture(scope="module")
+def ops(mta):
+    mta._native.load()
+    return torch.ops.mega_trading_amd
+
+
+def meta(*shape, dtype=torch.float32, grad=True):
+    return torch.empty(*shape, dtype=dtype, device="meta", requires_grad=grad)
+
+
+def tables():
+    return meta(8, 16, grad=False), meta(8, 16, grad=False)
+
+
+def heads(n, t=8):
+    return meta(2, n, t, 32, dtype=BF16)
+
+
+NO_FORMULA = {
+    "gqa_attn_decode": lambda: (heads(4, 1), heads(2), heads(2), 5, 0.2),
+    "gqa_attn_decode_dev": lambda: (heads(4, 1), heads(2), heads(2), torch.ones(1, dtype=torch.int32, device="meta"), 0.2),
+    "decode_rope_append": lambda: (heads(4, 1), heads(2, 1), heads(2, 1), *tables(), 3, None,
+                                   heads(2).detach(), heads(2).detach()),
+    "gqa_attn_decode_append": lambda: (heads(4, 1), heads(2, 1), heads(2, 1), *tables(), 3, None, 4, None,
+                                       heads(2).detach(), heads(2).detach(), 0.2),
+    "linear_rows": lambda: (meta(4, 128), [meta(8, 128), meta(16, 128)]),
+    "linear_rows_gate": lambda: (meta(4, 128), meta(8, 128), meta(8, 128)),
+    "rms_norm_bwd": lambda: (meta(4, 16), meta(16), meta(4), meta(4, 16)),
+    "swiglu_bwd": lambda: (meta(4, 16), meta(4, 16), meta(4, 16)),
+    "scale_pair": lambda: (meta(4, 16), meta(16), torch.zeros((), device="meta", requires_grad=True)),
+}
+SECOND_ORDER = {
+    "gqa_attn_fwd": lambda: (heads(4), heads(2), heads(2), 0.2),
+    "gqa_rope_attn_fwd": lambda: (heads(4), heads(2), heads(2), *tables(), 0.2),
+    "rms_norm_fwd": lambda: (meta(4, 16), meta(16), 1e-5),
+    "add_rms_norm_fwd": lambda: (meta(4, 16), meta(4, 16), meta(16), 1e-5),
+    "rms_norm_fwd_mixed": lambda: (meta(4, 16), meta(16), 1e-5, 0),
+    "swiglu_fwd": lambda: (meta(4, 16), meta(4, 16)),
+    "swiglu_packed_fwd": lambda: (meta(4, 32),),
+}
+
+
+def call(op, args):
+    out = op(*args)
+    outs = out if isinstance(out, (tuple, list)) else (out,)
+    flat = [y for x in args for y in (x if isinstance(x, list) else [x])]
+    return outs, [x for x in flat if isinstance(x, torch.Tensor) and x.requires_grad]
+
+
+@pytest.mark.parametrize("name", sorted(NO_FORMULA))
+def test_a_gradient_through_an_op_without_a_formula_is_refused(ops, name):
+    outs, leaves = call(getattr(ops, name), NO_FORMULA[name]())
+    for out in outs:
+        assert out.requires_grad
+        with pytest.raises(RuntimeError, match="no autograd formula"):
+            torch.autograd.grad(out, leaves, torch.ones_like(out), allow_unused=True, retain_graph=True)
+    with torch.no_grad():
+        assert not call(getattr(ops, name), NO_FORMULA[name]())[0][0].requires_grad
+
+
+@pytest.mark.parametrize("name", sorted(SECOND_ORDER))
+def test_a_second_order_gradient_is_refused(ops, name):
+    outs, leaves = call(getattr(ops, name), SECOND_ORDER[name]())
+    first = torch.autograd.grad(outs[-2] if name == "add_rms_norm_fwd" else outs[0], leaves, torch.ones_like(outs[0]),
+                                create_graph=True)
+    for g in first:
+        with pytest.raises(RuntimeError, match="no autograd formula"):
+            torch.autograd.grad(g, leaves, torch.ones_like(g), allow_unused=True, retain_graph=True)
+
+
+def test_the_mixed_residual_norm_refuses_a_second_order_gradient(ops):
+    x, r, w = meta(4, 16, dtype=BF16), meta(4, 16), meta(16)
+    _res, y, _rstd = ops.add_rms_norm_fwd_mixed(x, r, w, 1e-5)
+    for g in torch.autograd.grad(y, (x, r, w), torch.ones_like(y), create_graph=True):
+        with pytest.raises(RuntimeError, match="no autograd formula"):
+            torch.autograd.grad(g, (x, r, w), torch.ones_like(g), allow_unused=True, retain_graph=True)
+
+
+def test_an_op_without_a_formula_refuses_forward_mode_and_functional_transforms(ops):
+    x, w = meta(4, 128), meta(8, 128)
+    with torch.autograd.forward_ad.dual_level(), pytest.raises(RuntimeError, match="forward-mode"):
+        ops.linear_rows(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)), [w])
+    with pytest.raises(RuntimeError, match="functorch"):
+        torch.func.grad(lambda z: ops.linear_rows(z, [w.detach()]).sum())(x.detach())
+
+
+def test_integer_outputs_carry_no_gradient(ops):
+    assert not ops.topk_sample(meta(4, 128), meta(4, 128, grad=False), 3).requires_grad
