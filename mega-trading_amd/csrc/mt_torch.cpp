@@ -760,7 +760,8 @@ struct RopeFn : torch::autograd::Function<RopeFn> {
   }
 };
 
-// The gradients are computed in the forward and scaled here.
+// The gradients are computed in the forward and scaled here; they are linear in
+// the incoming one, and differentiable in it.
 using CeSig = std::tuple<at::Tensor, at::Tensor, at::Tensor>(const at::Tensor&, const at::Tensor&, const at::Tensor&,
                                                              int64_t, int64_t, bool);
 struct LinearCeFn : torch::autograd::Function<LinearCeFn> {
@@ -778,8 +779,14 @@ struct LinearCeFn : torch::autograd::Function<LinearCeFn> {
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     if (!g[0].defined() || !ctx->saved_data["need_grad"].toBool()) return variable_list(6);
     const auto s = ctx->get_saved_variables();
-    static const auto op = MT_OP(scale_pair);
     variable_list r(6);
+    if ((c10::GradMode::is_enabled() && g[0].requires_grad()) || g[0]._fw_grad(0).defined()) {
+      // products that a derivative with respect to the incoming gradient goes through
+      r[0] = s[0] * g[0].to(s[0].scalar_type());
+      r[1] = s[1] * g[0].to(s[1].scalar_type());
+      return r;
+    }
+    static const auto op = MT_OP(scale_pair);
     std::tie(r[0], r[1]) = op.call(s[0], s[1], g[0]);
     return r;
   }

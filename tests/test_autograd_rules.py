@@ -100,3 +100,23 @@ def test_an_op_without_a_formula_refuses_forward_mode_and_functional_transforms(
 
 def test_integer_outputs_carry_no_gradient(ops):
     assert not ops.topk_sample(meta(4, 128), meta(4, 128, grad=False), 3).requires_grad
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, BF16])
+def test_the_loss_head_is_differentiable_in_its_incoming_gradient(ops, dtype):
+    h, w, lam = meta(8, 16, dtype=dtype), meta(24, 16, dtype=dtype), torch.zeros((), device="meta", requires_grad=True)
+    labels = torch.zeros(8, dtype=torch.long, device="meta")
+    loss = lam * ops.fused_linear_ce(h, w, labels, -100, 2 if dtype == torch.float32 else 0, True)[0]
+    for g in torch.autograd.grad(loss, (h, w), create_graph=True):
+        (dlam,) = torch.autograd.grad(g.float().square().sum(), (lam,), retain_graph=True)
+        assert dlam.shape == ()
+
+
+def test_the_loss_head_passes_a_forward_mode_tangent_of_its_incoming_gradient(ops):
+    h, w = meta(8, 16), meta(24, 16)
+    loss = ops.fused_linear_ce(h, w, torch.zeros(8, dtype=torch.long, device="meta"), -100, 2, True)[0]
+    fw = torch.autograd.forward_ad
+    with fw.dual_level():
+        up = fw.make_dual(torch.ones((), device="meta"), torch.ones((), device="meta"))
+        for g in torch.autograd.grad(loss, (h, w), up):
+            assert fw.unpack_dual(g).tangent is not None

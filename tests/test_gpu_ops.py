@@ -572,3 +572,23 @@ def test_add_rms_norm_backward_row_pipeline(rows, dim, dt):
     tol = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -10, torch.float32: 2e-6}[dt]
     for a, b in ((got[0], ds), (got[1], ds), (got[2], dw)):
         assert float((a.double() - b).norm() / b.norm()) <= tol
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_loss_head_gradient_penalty(dt):
+    """d / d lam of |d (lam loss) / d hidden|^2 and of the same for the weight: 2 lam |d loss / d .|^2, and the plain
+    gradients are the penalty's first-order ones."""
+    ops = importlib.import_module("mega-trading_amd.ops")
+    g = torch.Generator(device="cuda").manual_seed(3)
+    h = torch.randn(40, 64, generator=g, device="cuda").to(dt).requires_grad_(True)
+    w = (torch.randn(96, 64, generator=g, device="cuda") / 8).to(dt).requires_grad_(True)
+    labels = torch.randint(0, 96, (40,), generator=g, device="cuda")
+    lam = torch.tensor(1.75, device="cuda", requires_grad=True)  # exact in 16 bits: both forms round once
+    plain = torch.autograd.grad(lam.detach() * ops.fused_linear_cross_entropy(h, w, labels), (h, w))
+    first = torch.autograd.grad(lam * ops.fused_linear_cross_entropy(h, w, labels), (h, w), create_graph=True)
+    for a, b in zip(first, plain):
+        assert torch.equal(a, b)
+        (got,) = torch.autograd.grad(a.float().square().sum(), (lam,), retain_graph=True)
+        want = 2 / 1.75 * float(b.double().square().sum())
+        # the 16-bit products and their sum are each rounded to 2^-9
+        assert abs(float(got) - want) <= (1e-5 if dt == torch.float32 else 2.0 ** -7) * want
