@@ -23,6 +23,7 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/variable.h>
 #include <torch/library.h>
 
 #include <array>
@@ -916,6 +917,24 @@ void no_formula(const c10::OperatorHandle& op, c10::DispatchKeySet ks, torch::ji
       torch::autograd::set_history(r.toTensor(), node);
 }
 
+// An op that writes caches counts it in their versions, so that a backward over
+// a cache saved before the write raises.  (torch's own fallback for this key only
+// looks at arguments that are returned.)
+void count_writes(const c10::OperatorHandle& op, c10::DispatchKeySet ks, torch::jit::Stack* stack) {
+  const auto& params = op.schema().arguments();
+  variable_list written;
+  for (size_t i = 0; i < params.size(); ++i) {
+    const c10::IValue& a = torch::jit::peek(*stack, i, params.size());
+    if (params[i].alias_info() && params[i].alias_info()->isWrite() && a.isTensor()) written.push_back(a.toTensor());
+  }
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    op.redispatchBoxed(ks & c10::after_ADInplaceOrView_keyset, stack);
+  }
+  for (const at::Tensor& t : written)
+    if (!t.is_inference()) torch::autograd::impl::bump_version(t);
+}
+
 }  // namespace
 
 TORCH_LIBRARY_IMPL(mega_trading_amd, Autograd, m) {
@@ -935,6 +954,11 @@ TORCH_LIBRARY_IMPL(mega_trading_amd, Autograd, m) {
   m.impl("swiglu_fwd", &swiglu_fwd_ad);
   m.impl("swiglu_packed_fwd", &swiglu_packed_fwd_ad);
   m.impl("rope_fwd", &rope_fwd_ad);
+}
+
+TORCH_LIBRARY_IMPL(mega_trading_amd, ADInplaceOrView, m) {
+  for (const char* op : {"decode_rope_append", "gqa_attn_decode_append"})
+    m.impl(op, torch::CppFunction::makeFromBoxedFunction<&count_writes>());
 }
 
 TORCH_LIBRARY_IMPL(mega_trading_amd, CUDA, m) {

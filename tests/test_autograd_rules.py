@@ -120,3 +120,35 @@ def test_the_loss_head_passes_a_forward_mode_tangent_of_its_incoming_gradient(op
         up = fw.make_dual(torch.ones((), device="meta"), torch.ones((), device="meta"))
         for g in torch.autograd.grad(loss, (h, w), up):
             assert fw.unpack_dual(g).tangent is not None
+
+
+def append_args(name, grad, base=None):
+    caches = list(base) if base is not None else [heads(2).detach(), heads(2).detach()]
+    new = [x if grad else x.detach() for x in (heads(4, 1), heads(2, 1), heads(2, 1))]
+    return (*new, *tables(), 3, None, *((4, None) if name == "gqa_attn_decode_append" else ()), *caches,
+            *((0.2,) if name == "gqa_attn_decode_append" else ())), caches
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("name", ["decode_rope_append", "gqa_attn_decode_append"])
+def test_an_append_counts_as_a_write_to_the_caches(ops, name, grad):
+    args, caches = append_args(name, grad)
+    out = getattr(ops, name)(*args)
+    assert [c._version for c in caches] == [1, 1] and out._version == 0
+    assert not any(c.requires_grad for c in caches)
+    both = meta(2, 2, 2, 8, 32, dtype=BF16, grad=False)  # the layers' caches as views of one tensor
+    getattr(ops, name)(*append_args(name, grad, (both[0], both[1]))[0])
+    assert both._version == 2
+    with torch.inference_mode():  # inference tensors have no versions
+        inference = [c.clone() for c in caches]
+        getattr(ops, name)(*append_args(name, False, inference)[0])
+    getattr(ops, name)(*append_args(name, False, inference)[0])
+
+
+@pytest.mark.parametrize("name", ["decode_rope_append", "gqa_attn_decode_append"])
+def test_a_cache_saved_for_backward_and_then_written_is_noticed(ops, name):
+    args, (k_cache, _v_cache) = append_args(name, False)
+    y = (k_cache * heads(2)).sum()
+    getattr(ops, name)(*args)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.backward()
