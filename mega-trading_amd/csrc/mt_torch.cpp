@@ -793,7 +793,8 @@ struct LinearCeFn : torch::autograd::Function<LinearCeFn> {
   }
 };
 
-// Whether a call records a gradient: without one the op runs below autograd directly.
+// Whether a call records a gradient: without one the op runs below autograd
+// directly.  RoPE tables that require one record the call too (and get none).
 template <class... T>
 bool records(const T&... ts) {
   return c10::GradMode::is_enabled() && (ts.requires_grad() || ...);
@@ -816,7 +817,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> gqa_rope_attn_fwd_ad(
                                                                                 const at::Tensor& v,
                                                                                 const at::Tensor& cos,
                                                                                 const at::Tensor& sin, double scale) {
-  if (!records(q, k, v)) MT_BELOW(gqa_rope_attn_fwd, q, k, v, cos, sin, scale);
+  if (!records(q, k, v, cos, sin)) MT_BELOW(gqa_rope_attn_fwd, q, k, v, cos, sin, scale);
   auto r = RopeAttnFn::apply(q, k, v, cos, sin, scale);
   return {r[0], r[1], r[2], r[3]};
 }
@@ -825,7 +826,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> gqa_rope_attn_packed_
                                                                                        const at::Tensor& sin,
                                                                                        int64_t hq, int64_t hkv,
                                                                                        double scale) {
-  if (!records(qkv)) MT_BELOW(gqa_rope_attn_packed_fwd, qkv, cos, sin, hq, hkv, scale);
+  if (!records(qkv, cos, sin)) MT_BELOW(gqa_rope_attn_packed_fwd, qkv, cos, sin, hq, hkv, scale);
   auto r = PackedAttnFn::apply(qkv, cos, sin, hq, hkv, scale);
   return {r[0], r[1], r[2], r[3]};
 }
@@ -862,7 +863,7 @@ at::Tensor swiglu_packed_fwd_ad(const at::Tensor& gate_up) {
 }
 std::tuple<at::Tensor, at::Tensor> rope_fwd_ad(const at::Tensor& q, const at::Tensor& k, const at::Tensor& cos,
                                                const at::Tensor& sin, bool inverse) {
-  if (!records(q, k)) MT_BELOW(rope_fwd, q, k, cos, sin, inverse);
+  if (!records(q, k, cos, sin)) MT_BELOW(rope_fwd, q, k, cos, sin, inverse);
   auto r = RopeFn::apply(q, k, cos, sin, inverse);
   return {r[0], r[1]};
 }

@@ -152,3 +152,14 @@ def test_a_cache_saved_for_backward_and_then_written_is_noticed(ops, name):
     getattr(ops, name)(*args)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         y.backward()
+
+
+@pytest.mark.parametrize("name", ["gqa_rope_attn_fwd", "gqa_rope_attn_packed_fwd", "rope_fwd"])
+def test_a_call_whose_tables_alone_require_a_gradient_is_recorded(ops, name):
+    cos, sin = meta(8, 16), meta(8, 16, grad=False)
+    q, k = heads(4).detach(), heads(2).detach()
+    args = {"gqa_rope_attn_fwd": (q, k, k, cos, sin, 0.2), "rope_fwd": (q, k, cos, sin, False),
+            "gqa_rope_attn_packed_fwd": (meta(2, 8, 8 * 32, dtype=BF16, grad=False), cos, sin, 4, 2, 0.2)}[name]
+    out = getattr(ops, name)(*args)[0]
+    assert out.requires_grad
+    assert torch.autograd.grad(out, cos, torch.ones_like(out), allow_unused=True) == (None,)
