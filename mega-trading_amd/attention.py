@@ -264,7 +264,8 @@ def decode_append_attention(query: torch.Tensor, key: torch.Tensor, value: torch
     """``decode_rope_append`` then ``decode_attention`` on its rotated query:
     the same arguments, checks and values.  Where the kernels can load the new
     rows 16 bytes at a time and a group has at most 8 query heads it is one
-    launch pair (``mt_gqa_attn_decode_append``) instead of two calls."""
+    launch pair (``mt_gqa_attn_decode_append``) instead of two calls.  (The op
+    itself looks at the addresses, which a tracer's tensors do not have.)"""
     dev = isinstance(pos, torch.Tensor)
     b, hq, _, d = query.shape
     unit = 4 if query.dtype == torch.float32 else 8
@@ -273,7 +274,6 @@ def decode_append_attention(query: torch.Tensor, key: torch.Tensor, value: torch
              and (dev or 0 <= pos < key_cache.shape[2] and 1 <= length <= key_cache.shape[2])
              and cos.dtype == torch.float32 and sin.dtype == torch.float32 and cos.is_contiguous() and sin.is_contiguous()
              and cos.shape == sin.shape
-             and all(t.data_ptr() % 16 == 0 for t in (query, key, value, cos, sin, key_cache, value_cache))
              and all(st % unit == 0 for t in (query, key, value) for st in t.stride()[:2])
              and all(st % 8 == 0 for t in (key_cache, value_cache) for st in t.stride()[:3]))
     if not fused:

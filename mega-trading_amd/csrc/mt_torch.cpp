@@ -36,8 +36,10 @@
 
 namespace {
 
+bool aligned16(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
 bool kernel_ready(const at::Tensor& t) {
-  if (t.dim() == 0 || t.stride(-1) != 1 || reinterpret_cast<uintptr_t>(t.data_ptr()) % 16) return false;
+  if (t.dim() == 0 || t.stride(-1) != 1 || !aligned16(t)) return false;
   for (int64_t i = 0; i + 1 < t.dim(); ++i)
     if (t.size(i) > 1 && t.stride(i) % 8) return false;
   return true;
@@ -257,6 +259,12 @@ at::Tensor gqa_attn_decode_append(const at::Tensor& q, const at::Tensor& k, cons
                                   int64_t length, const std::optional<at::Tensor>& length_dev,
                                   const at::Tensor& k_cache, const at::Tensor& v_cache, double scale) {
   const c10::DeviceGuard guard(q.device());
+  // rows that cannot be loaded 16 bytes at a time: the two launches it stands for
+  for (const at::Tensor* t : {&q, &k, &v, &cos, &sin, &k_cache, &v_cache})
+    if (!aligned16(*t)) {
+      const at::Tensor q_rot = decode_rope_append(q, k, v, cos, sin, pos, pos_dev, k_cache, v_cache);
+      return decode(q_rot, k_cache, v_cache, length, int_ptr_or_null(length_dev), scale);
+    }
   const int64_t b = q.size(0), hq = q.size(1), d = q.size(3), hkv = k_cache.size(1), cap = k_cache.size(2);
   const at::Tensor out = at::empty({b, hq, 1, d}, k_cache.options());
   const int* len = int_ptr_or_null(length_dev);
@@ -274,8 +282,6 @@ at::Tensor gqa_attn_decode_append(const at::Tensor& q, const at::Tensor& k, cons
 }
 
 // --- row operators (schemas in ops.py, projection.py) ------------------------
-bool aligned16(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
-
 at::Tensor flat(const at::Tensor& x) {
   const at::Tensor c = x.contiguous();
   return aligned16(c) ? c : c.clone();

@@ -377,3 +377,20 @@ def test_decode_rope_append_bounds_pos_before_launch(mta):
     assert call(0, 0, 40) == -2
     assert lib.mt_decode_rope_append(p, p, p, ins, p, p, 64, 3, None, p, p, p, cst, 40, 1, 8, 2, 64, 0, 2,
                                      None) == -4  # fp32 caches
+
+
+@pytest.mark.parametrize("dev", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_the_decode_step_traces_as_one_graph(dtype, dev):
+    import importlib
+
+    attn = importlib.import_module("mega-trading_amd.attention")
+    torch._dynamo.reset()
+    with FakeTensorMode(), torch.no_grad():
+        q, k, v = (_fake((2, n, 1, 64), dtype) for n in (8, 2, 2))
+        kc, vc = _fake((2, 2, 40, 64)), _fake((2, 2, 40, 64))
+        table = _fake((40, 32), torch.float32)
+        pos, length = (torch.zeros(1, device="cuda", dtype=torch.int32) for _ in range(2)) if dev else (3, 4)
+        step = torch.compile(attn.decode_append_attention, fullgraph=True, backend="eager")
+        out = step(q, k, v, table, table, pos, length, kc, vc, repeats=4)
+    assert out.shape == q.shape and out.dtype == kc.dtype

@@ -386,3 +386,34 @@ def test_decode_append_attention_equals_the_two_calls(b, hq, hkv, d, cap, pos, i
                                     repeats=hq // hkv)
         got = attn.decode_append_attention(q, k, v, rope.cos, rope.sin, at, n, k2, v2, repeats=hq // hkv)
         assert torch.equal(k1, k2) and torch.equal(v1, v2) and torch.equal(ref, got), length
+
+
+@pytest.mark.parametrize("which", ["query", "value", "cos", "value_cache"])
+@pytest.mark.parametrize("dev", [False, True])
+def test_decode_append_attention_takes_misaligned_tensors(which, dev):
+    """A tensor that starts 8 bytes past a 16-byte boundary: the values of the two calls, which refuse such
+    a table or cache."""
+    attn = importlib.import_module("mega-trading_amd.attention")
+    b, hq, hkv, d, cap, pos = 3, 8, 2, 64, 80, 66
+
+    def place(t, name):
+        if name != which:
+            return t.cuda()
+        shift = 8 // t.element_size()
+        flat = torch.empty(t.numel() + shift, dtype=t.dtype, device="cuda")[shift:]
+        return flat.copy_(t.reshape(-1)).view(t.shape)
+
+    g = torch.Generator().manual_seed(11)
+    rope = model_mod.RotaryEmbedding(d, cap, theta=10_000.0)
+    q, k, v = (place(torch.randn(b, n, 1, d, generator=g), name) for n, name in ((hq, "query"), (hkv, "key"), (hkv, "value")))
+    cos, sin = place(rope.cos, "cos"), rope.sin.cuda()
+    kc, vc = (torch.randn(b, hkv, cap, d, generator=g).bfloat16() for _ in range(2))
+    at, n = ((torch.tensor([x], dtype=torch.int32, device="cuda") for x in (pos, pos + 1)) if dev else (pos, pos + 1))
+    k1, v1, k2, v2 = place(kc, "key_cache"), place(vc, "value_cache"), kc.cuda(), vc.cuda()
+    if which in ("cos", "value_cache"):
+        with pytest.raises(RuntimeError, match="16-byte aligned"):
+            attn.decode_append_attention(q, k, v, cos, sin, at, n, k1, v1, repeats=hq // hkv)
+        return
+    got = attn.decode_append_attention(q, k, v, cos, sin, at, n, k1, v1, repeats=hq // hkv)
+    ref = attn.decode_attention(attn.decode_rope_append(q, k, v, cos, sin, at, k2, v2), k2, v2, n, repeats=hq // hkv)
+    assert torch.equal(k1, k2) and torch.equal(v1, v2) and torch.equal(got, ref)
