@@ -178,13 +178,13 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(DecodeParams p) {
 #pragma unroll
       for (int c = 0; c < Ly::KS; ++c) qf[c] = *reinterpret_cast<const u32x4*>(qb + 32 * c);
     }
-    if (owner) {
+    if (owner) {  // every load of the new row, also those of keys past the end: the cache may still hold the old one
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int c = 0; c < Ly::KS; ++c) kw[t][c] = 16 * t + hn == pos - k0 ? knew[c] : kw[t][c];
+        for (int c = 0; c < Ly::KS; ++c) kw[t][c] = min(16 * t + hn, n - 1) == pos - k0 ? knew[c] : kw[t][c];
 #pragma unroll
-      for (int i = 0; i < Ly::NV; ++i) vw[i] = kg + i * Ly::G == pos - k0 ? vnew : vw[i];
+      for (int i = 0; i < Ly::NV; ++i) vw[i] = min(kg + i * Ly::G, n - 1) == pos - k0 ? vnew : vw[i];
     }
     f32x4 sc[4];
 #pragma unroll

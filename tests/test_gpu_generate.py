@@ -381,7 +381,7 @@ def test_decode_append_attention_equals_the_two_calls(b, hq, hkv, d, cap, pos, i
     for length in {pos + 1, max(1, pos // 2), min(cap, pos + 70)}:  # also lengths that are not pos + 1
         n = torch.tensor([length], dtype=torch.int32, device="cuda") if dev else length
         k1, v1, k2, v2 = kc.clone(), vc.clone(), kc.clone(), vc.clone()
-        k2[:, :, pos] = float("nan")  # the stale row is never used
+        k2[:, :, pos] = v2[:, :, pos] = float("nan")  # the stale rows are never used
         ref = attn.decode_attention(attn.decode_rope_append(q, k, v, rope.cos, rope.sin, at, k1, v1), k1, v1, n,
                                     repeats=hq // hkv)
         got = attn.decode_append_attention(q, k, v, rope.cos, rope.sin, at, n, k2, v2, repeats=hq // hkv)
