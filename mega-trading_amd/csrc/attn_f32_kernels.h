@@ -197,6 +197,9 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_fwd_f32_kernel(Attn
     }
     reads_done();
     if (more) kst.stage(K, kbase, p.sk[2], (kt + SPLIT) * 32, p.T);
+    // scaled before the mask: any scale, 0 and negative ones too, leaves -inf as it is
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] *= c2;
     if (kt == task.blk) {  // the diagonal; tiles left of it have every key <= every row
 #pragma unroll
       for (int i = 0; i < 16; ++i)
@@ -205,10 +208,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_fwd_f32_kernel(Attn
     // the diagonal tile holds key 32 kt <= row, so m is finite after a wave's first tile
     float mx = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      s[i] *= c2;
-      mx = fmaxf(mx, s[i]);
-    }
+    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
     const float mnew = fmaxf(m, max_with_partner(mx));
     const float alpha = exp2_fast(m - mnew);
     float ps = 0.f;

@@ -418,3 +418,26 @@ def test_small_grids_split_keys_over_waves(b, t, hq, hkv, d, dt):
     pkg = importlib.import_module("mega-trading_amd")
     compare(run_hip(pkg, q, k, v, do, hq // hkv), oracle(q, k, v, do, hq // hkv))
     compare(run_hip(pkg, q, k, v, do, hq // hkv, cos, sin), oracle(q, k, v, do, hq // hkv, cos, sin))
+
+
+@pytest.mark.parametrize("b,t,hq,hkv,d", [(1, 70, 4, 2, 64), (64, 40, 32, 32, 32)])  # tiles dealt to waves, row blocks a wave
+@pytest.mark.parametrize("scale", [0.0, -0.3])
+def test_fp32_kernels_take_any_scale(b, t, hq, hkv, d, scale):
+    """Forward, LSE and backward at a scale of 0 (the mean of the visible rows) and a negative one, against float64;
+    the bound as in test_fp32_tile_edges_and_both_forward_forms."""
+    importlib.import_module("mega-trading_amd._native").ensure()
+    g = torch.Generator(device="cuda").manual_seed(t)
+    q, do = (torch.randn(b, hq, t, d, generator=g, device="cuda") for _ in range(2))
+    k, v = (torch.randn(b, hkv, t, d, generator=g, device="cuda") for _ in range(2))
+    args = [x.requires_grad_(True) for x in (q, k, v)]
+    out, lse = torch.ops.mega_trading_amd.gqa_attn_fwd(*args, scale)
+    got = (out, lse, *torch.autograd.grad(out, args, do))
+    ref_in = [x.detach().double().requires_grad_(True) for x in args]
+    kk, vv = (x.repeat_interleave(hq // hkv, dim=1) for x in ref_in[1:])
+    s = (ref_in[0] @ kk.transpose(2, 3) * scale).masked_fill(
+        torch.ones(t, t, dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+    ref = torch.softmax(s, dim=-1) @ vv
+    refs = (ref, torch.logsumexp(s, dim=-1), *torch.autograd.grad(ref, ref_in, do.double()))
+    for a, r in zip(got, refs):
+        err = float((a.detach().double() - r.detach()).norm() / max(float(r.detach().norm()), r.numel() ** 0.5))
+        assert err <= (t + d) * 2.0 ** -24, err
