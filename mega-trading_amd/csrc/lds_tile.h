@@ -117,9 +117,10 @@ __device__ __forceinline__ uint32_t lds_addr(const void* l) {
   return (uint32_t)(uintptr_t)l;
 }
 
-__device__ __forceinline__ void lds_dma16(const uint16_t* g, char* l) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "{m0}"(lds_addr(l)));
+__device__ __forceinline__ void lds_dma16(const void* g, uint32_t l) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "{m0}"(l));
 }
+__device__ __forceinline__ void lds_dma16(const void* g, char* l) { lds_dma16(g, lds_addr(l)); }
 
 __device__ __forceinline__ void lds_dma4(const float* g, char* l) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "{m0}"(lds_addr(l)));
@@ -198,53 +199,59 @@ struct Stager {
 };
 
 // Copies of ROWS rows by one wave into LDS of its own (lds wave-uniform), W the
-// row width in 16-bit values, T the element type of the matrix: the offsets of
-// 16 rows, the swizzle's period, are kept and the scalar base moves for the
-// others.  The wave waits for them by count (copies_done), with no barrier.
+// row width in 16-bit values, T the element type of the matrix.  A 1 KB copy is
+// RPC whole rows; its chunks differ from the first copy's by an exclusive or (the
+// swizzle's row bits of the copy and of the lane do not overlap).  Up to 4 copies
+// per 16 rows, the swizzle's period, their offsets are kept and the scalar base
+// moves for the other rows; more of them (D = 128 fp32: 8 for each of two
+// matrices) push attn_bwd_dkv_f32_kernel into scratch, whose reloads wait for the
+// copies, so there the offsets are formed at each copy and the scalar base moves
+// for every one.  fp32 forward + backward with RoPE, kept / formed, us: 2 x 1024, 16
+// / 4 heads of 128 660 / 629, 1 x 2000 1230 / 1114; of 64, 8 x 512 239 / 253, 4 x
+// 1000, 8 / 2 heads 284 / 298.  The wave waits for its copies by count
+// (copies_done), with no barrier.
 template <class T, int W, int ROWS>
 struct WaveStager {
   using TL = Tile<W>;
-  static constexpr int G = ROWS / 16;
-  static constexpr int N = TL::NC / 4;       // 1 KB copies of 16 rows
-  static constexpr int COPIES = G * N;       // of a tile, whatever path it takes
+  static constexpr int RPC = 64 / TL::NC;    // rows of a copy
+  static constexpr int COPIES = ROWS / RPC;  // of a tile, whatever path it takes
+  static constexpr int N = 16 / RPC;         // copies of 16 rows
+  static constexpr bool KEPT = N <= 4;
   static constexpr int EL = 16 / sizeof(T);  // elements per 16-byte chunk
-  uint32_t voff[N];
-  int lane_;
+  static_assert(ROWS % 16 == 0, "the swizzle's period");
+  uint32_t voff[KEPT ? N : 1];  // bytes from the first row of 16; not KEPT: of the lane's row in a copy
+  int chunk;                    // of the lane in the first copy
 
-  static __device__ __forceinline__ void place(int i, int lane, int& row, int& chunk) {
-    const int f = i * 64 + lane;
-    row = f / TL::NC;
-    chunk = (f % TL::NC) ^ TL::swz(row);
-  }
   __device__ __forceinline__ void init(int64_t row_stride, int lane) {
+    const int r = lane / TL::NC;
+    chunk = (lane % TL::NC) ^ TL::swz(r);
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      int row, chunk;
-      place(i, lane, row, chunk);
-      voff[i] = (uint32_t)(row * (int)row_stride + chunk * EL) * (uint32_t)sizeof(T);
-    }
-    lane_ = lane;
+    for (int i = 0; i < (KEPT ? N : 1); ++i)
+      voff[i] = (uint32_t)((i * RPC + r) * (int)row_stride + (KEPT ? (chunk ^ TL::swz(i * RPC)) * EL : 0)) *
+                (uint32_t)sizeof(T);
   }
   // rows [row0, row0 + ROWS) of the matrix at src; rows past T_ - 1 copy row T_ - 1
   __device__ __forceinline__ void stage(char* lds, const T* src, int64_t row_stride, int row0, int T_) const {
+    uint32_t l0 = lds_addr(lds);
+    int ch = chunk;
+    // what is formed here is not kept in registers across the loop around the call
+    if constexpr (!KEPT) asm volatile("" : "+s"(l0), "+v"(ch));
     if (row0 + ROWS <= T_) {
-      const uint32_t l0 = lds_addr(lds);
 #pragma unroll
-      for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int i = 0; i < N; ++i)
-          lds_dma16_s(src + (int64_t)(row0 + 16 * g) * row_stride, voff[i], l0 + (g * N + i) * 1024);
+      for (int c = 0; c < COPIES; ++c) {
+        if constexpr (KEPT)
+          lds_dma16_s(src + (int64_t)(row0 + c / N * 16) * row_stride, voff[c % N], l0 + c * 1024);
+        else
+          lds_dma16_s(src + (int64_t)(row0 + c * RPC) * row_stride, voff[0] + ((uint32_t)(ch ^ TL::swz(c * RPC)) << 4),
+                      l0 + c * 1024);
+      }
     } else {
+      const int r = (int)(threadIdx.x & 63) / TL::NC;
 #pragma unroll
-      for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          int row, chunk;
-          place(i, lane_, row, chunk);
-          const int grow = min(row0 + 16 * g + row, T_ - 1);
-          lds_dma16(reinterpret_cast<const uint16_t*>(src + (int64_t)grow * row_stride + chunk * EL),
-                    lds + (g * N + i) * 1024);
-        }
+      for (int c = 0; c < COPIES; ++c) {
+        const int grow = min(row0 + c * RPC + r, T_ - 1);
+        lds_dma16(src + (int64_t)grow * row_stride + (ch ^ TL::swz(c * RPC)) * EL, l0 + c * 1024);
+      }
     }
   }
 };

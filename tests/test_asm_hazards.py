@@ -133,3 +133,21 @@ def test_wave_private_and_split_copies_have_their_wait_states(tmp_path):
     ins = _instructions(out.read_text())
     test_every_lds_copy_has_its_wait_states(ins)
     assert not [x for x in ins if x.startswith("v_") and _writes(x, {"m0"})]
+
+
+def test_fp32_kernels_use_no_scratch(tmp_path):
+    """A spill in the fp32 loops would be reloaded between the copies in flight, each reload waiting for all of them."""
+    hipcc = _hipcc()
+    if hipcc is None:
+        pytest.skip("hipcc not available")
+    src, out = tmp_path / "tu.hip", tmp_path / "tu.s"
+    src.write_text('#include "attn_f32_kernels.h"\n' + "".join(
+        f"template __global__ void mt::{k}(mt::AttnParams);\n" for d in (32, 64, 128) for k in (
+            f"attn_fwd_f32_kernel<{d}, true, 1>", f"attn_fwd_f32_kernel<{d}, true, 4>", f"attn_bwd_dq_f32_kernel<{d}, true, 1>",
+            f"attn_bwd_dq_f32_kernel<{d}, true, 4>", f"attn_bwd_dkv_f32_kernel<{d}, true>", f"attn_bwd_dkv_f32_kernel<{d}, false>")))
+    proc = subprocess.run([hipcc, "--offload-arch=gfx950", "-O3", "-std=c++17", "--cuda-device-only", "-S",
+                           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-pass-failed",
+                           "-I", CSRC, str(src), "-o", str(out)], capture_output=True, text=True, timeout=900)
+    assert proc.returncode == 0, proc.stderr[-2000:]
+    sizes = re.findall(r"; ScratchSize: (\d+)", out.read_text())
+    assert len(sizes) == 18 and set(sizes) == {"0"}
