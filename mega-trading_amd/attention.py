@@ -397,8 +397,9 @@ def _forward_padded(q, k, v, cos, sin, dk):
         out, lse = _attn_fwd(qp, kp, vp, scale)
     else:
         half = (dk - d) // 2
-        cos = F.pad(cos, (0, half), value=1.0)
-        sin = F.pad(sin, (0, half), value=0.0)
+        rows = q.shape[2]  # of a table that may be far longer
+        cos = F.pad(cos.reshape(-1, d // 2)[:rows], (0, half), value=1.0)
+        sin = F.pad(sin.reshape(-1, d // 2)[:rows], (0, half), value=0.0)
         out, lse, _q_rot, _k_rot = _rope_attn_fwd(qp, kp, vp, cos, sin, scale)
     result = torch.empty_like(q)
     result.copy_(out[..., :d])

@@ -394,3 +394,21 @@ def test_the_decode_step_traces_as_one_graph(dtype, dev):
         step = torch.compile(attn.decode_append_attention, fullgraph=True, backend="eager")
         out = step(q, k, v, table, table, pos, length, kc, vc, repeats=4)
     assert out.shape == q.shape and out.dtype == kc.dtype
+
+
+def test_a_padded_head_size_pads_only_the_rows_of_the_tables_it_reads(mta):
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    seen = []
+
+    class Tables(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if func is torch.ops.mega_trading_amd.gqa_rope_attn_fwd.default:
+                seen.extend(tuple(t.shape) for t in args[3:5])
+            return func(*args, **(kwargs or {}))
+
+    with FakeTensorMode(), Tables():
+        q, k = _fake((2, 4, 16, 48)), _fake((2, 2, 16, 48))
+        table = _fake((1, 1, 4096, 24), torch.float32)
+        mta.rope_attention(q, k, k, table, table, repeats=2)
+    assert seen == [(16, 32), (16, 32)]
