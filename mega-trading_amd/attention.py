@@ -220,10 +220,8 @@ def decode_rope_append(query: torch.Tensor, key: torch.Tensor, value: torch.Tens
     cos, sin = cos.to(torch.float32), sin.to(torch.float32)
     _native.ensure()
     if isinstance(pos, torch.Tensor):
-        return _rope_append(query, key, value, cos, sin, last, pos, key_cache,
-                                                             value_cache)
-    return _rope_append(query, key, value, cos, sin, int(pos), None, key_cache,
-                                                         value_cache)
+        return _rope_append(query, key, value, cos, sin, last, pos, key_cache, value_cache)
+    return _rope_append(query, key, value, cos, sin, int(pos), None, key_cache, value_cache)
 
 
 def _check_append(query, key, value, cos, sin, pos, key_cache, value_cache) -> int:
@@ -289,10 +287,9 @@ def decode_append_attention(query: torch.Tensor, key: torch.Tensor, value: torch
     if dev:
         if length.dtype != torch.int32 or length.numel() != 1 or length.device != query.device:
             raise ValueError("a tensor length must be a one-element int32 tensor on the query's device")
-        return _attn_decode_append(query, key, value, cos, sin, last, pos, 0, length,
-                                                                 key_cache, value_cache, scale)
-    return _attn_decode_append(query, key, value, cos, sin, int(pos), None, int(length),
-                                                             None, key_cache, value_cache, scale)
+        return _attn_decode_append(query, key, value, cos, sin, last, pos, 0, length, key_cache, value_cache, scale)
+    return _attn_decode_append(query, key, value, cos, sin, int(pos), None, int(length), None, key_cache, value_cache,
+                               scale)
 
 
 # ---------------------------------------------------------------------------
@@ -337,30 +334,6 @@ def _rope_tables(cos: torch.Tensor, sin: torch.Tensor, query: torch.Tensor) -> t
         else:
             out.append(tab.reshape(-1, d // 2)[:t].to(device=query.device, dtype=torch.float32).contiguous())
     return out[0], out[1]
-
-
-def _kernel_ready(t: torch.Tensor) -> torch.Tensor:
-    """Unit last stride, 8-element-aligned outer strides and a 16-byte-aligned base."""
-    ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0
-    if ok:
-        for size, stride in zip(t.shape[:-1], t.stride()[:-1]):
-            if size > 1 and stride % 8:
-                ok = False
-                break
-    return t if ok else t.contiguous()
-
-
-def _strides(*tensors: torch.Tensor):
-    flat = []
-    for t in tensors:
-        flat.extend(int(st) if sz > 1 else 0 for sz, st in zip(t.shape, t.stride()))
-    import ctypes
-
-    return (ctypes.c_int64 * len(flat))(*flat)
-
-
-def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
-    return None if t is None else t.data_ptr()
 
 
 def _kernel_head_dim(d: int) -> int:

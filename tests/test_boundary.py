@@ -345,19 +345,6 @@ def test_fake_impls_give_shapes_for_tracing(mta):
         assert tok.shape == (32, 1) and tok.dtype == torch.int64
 
 
-def test_kernel_ready_keeps_model_layout_views():
-    """The [B,T,H,D]-physical views of model.py:220-222 pass through without a copy."""
-    import importlib
-
-    ops = importlib.import_module("mega-trading_amd.attention")
-    x = torch.randn(2, 16, 8, 64).transpose(1, 2)  # [B, H, T, D] view
-    assert ops._kernel_ready(x) is x
-    y = torch.randn(2, 8, 16, 64)[..., ::2]  # non-unit last stride -> copy
-    assert ops._kernel_ready(y).is_contiguous()
-    arr = ops._strides(torch.empty(1, 1, 5, 32))
-    assert list(arr) == [0, 0, 32, 1]  # size-1 dims pass stride 0
-
-
 def test_decode_rope_append_bounds_pos_before_launch(mta):
     """mt_decode_rope_append rejects a position at or past the cache capacity or
     the RoPE table before any launch (pointers never dereferenced)."""

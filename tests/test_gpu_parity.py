@@ -441,3 +441,40 @@ def test_fp32_kernels_take_any_scale(b, t, hq, hkv, d, scale):
     for a, r in zip(got, refs):
         err = float((a.detach().double() - r.detach()).norm() / max(float(r.detach().norm()), r.numel() ** 0.5))
         assert err <= (t + d) * 2.0 ** -24, err
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_which_layouts_are_read_in_place(mta, dt):
+    """The layout rule of the attention ops: [B, T, H, D]-physical views and size-1 dims with odd strides are read in
+    place (no more allocations than contiguous tensors take), other strides are copied, a misaligned contiguous
+    tensor is refused; the values are those of contiguous tensors."""
+    b, t, hq, hkv, d = 2, 70, 4, 2, 64
+    g = torch.Generator(device="cuda").manual_seed(5)
+
+    def run(q, k, v):
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        with torch.no_grad():
+            out = mta.attention(q, k, v, repeats=hq // hkv)
+        return out, torch.cuda.memory_stats()["allocation.all.allocated"] - before
+
+    plain = [torch.randn(b, h, t, d, generator=g, device="cuda").to(dt) for h in (hq, hkv, hkv)]
+    want, base = run(*plain)
+    wide = lambda x, n, s: torch.zeros(*x.shape[:-1], n, device="cuda", dtype=dt)[..., s:s + x.shape[-1]].copy_(x)  # noqa: E731
+    views = {
+        "model": [x.transpose(1, 2).contiguous().transpose(1, 2) for x in plain],
+        "slice": [wide(x, 80, 8) for x in plain],
+        "row stride": [wide(x, 68, 0) for x in plain],
+        "step": [x.repeat_interleave(2, dim=-1)[..., ::2] for x in plain],
+        "base": [wide(x, 72, 1) for x in plain],
+    }
+    for name, x in views.items():
+        got, allocs = run(*x)
+        assert torch.equal(got, want), name
+        assert (allocs == base) if name in ("model", "slice") else (allocs > base), (name, allocs, base)
+    one = [torch.empty_strided((1, h, t, d), (3, t * d, d, 1), device="cuda", dtype=dt).copy_(x[:1])
+           for h, x in zip((hq, hkv, hkv), plain)]  # a batch of 1: its stride is never used
+    got, allocs = run(*one)
+    assert torch.equal(got, want[:1]) and allocs == base
+    shifted = torch.empty(plain[0].numel() + 1, device="cuda", dtype=dt)[1:].view(plain[0].shape).copy_(plain[0])
+    with pytest.raises(RuntimeError, match="16-byte aligned"):
+        run(shifted, *plain[1:])
