@@ -18,7 +18,7 @@
 // memory, a row per lane with 16 bytes from each of 64 cache lines a load, the
 // same tiles left the MFMAs idle two thirds of the time.  Measured, forward +
 // backward with RoPE: 8 x 512, 16 / 4 heads of 64: 362 -> 238 us; 4 x 1000, 8 / 2
-// of 64: 441 -> 285; 2 x 1024, 16 / 4 of 128: 1086 -> 629; 2 x 256, 4 / 2 of 32:
+// of 64: 441 -> 285; 2 x 1024, 16 / 4 of 128: 1086 -> 605; 2 x 256, 4 / 2 of 32:
 // 48.6 -> 33.0.
 //
 // MFMA layout (32x32x2, fp32): A[m][k] comes from lane m + 32 k, B[k][n] from
@@ -88,8 +88,8 @@ __global__ __launch_bounds__(256) void rope_f32_kernel(const float* x, int64_t s
 // a row of 2 D 16-bit values (lds_tile.h).
 // ---------------------------------------------------------------------------
 // Copies of 32 rows by one wave (WaveStager, lds_tile.h).
-template <int D>
-using F32Stager = WaveStager<float, 2 * D, 32>;
+template <int D, bool KEPT = true>
+using F32Stager = WaveStager<float, 2 * D, 32, KEPT>;
 
 // Operand reads of such a tile.
 //  * row: lane (row l32, half hh) reads d values hh D/2 + 4 j .. + 3 (the score
@@ -118,8 +118,7 @@ struct F32Tile {
 
 // The values a wave loaded for itself are here.  Asked before a loop over copied
 // tiles: left to the first use, the compiler's wait stands inside the loop and
-// drains the copies in flight in every pass (4 x 1000, 8 / 2 heads of 64, forward +
-// backward: 291 us without, 285 with).
+// drains the copies in flight in every pass.
 template <int N>
 __device__ __forceinline__ void loads_done(const float (&v)[N]) {
 #pragma unroll
@@ -191,7 +190,6 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_fwd_f32_kernel(Attn
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) zero16(oacc[dt]);
   float m = -INFINITY, l = 0.f;
-  loads_done(qv);
   for (int kt = kt0; kt <= task.blk; kt += SPLIT) {
     const bool more = kt + SPLIT <= task.blk;
     // K is here; V may still be on its way (the first time the wave also has its
@@ -245,50 +243,50 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_fwd_f32_kernel(Attn
     if (more) vst.stage(V, vbase, p.sv[2], (kt + SPLIT) * 32, p.T);
   }
   if constexpr (SPLIT == 4) {
-  __syncthreads();  // every wave's tiles are read: the block is reused for the merge
-  // merge the four waves' (O, m, l) with the log-sum-exp rule (a wave that
-  // had no tile has m = -inf and contributes nothing); m is the same on a
-  // lane and its lane^32 partner
-  if (wave > 0) {
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-        red_o[wave - 1][dt * 4 + g][lane] =
-            f32x4{oacc[dt][4 * g], oacc[dt][4 * g + 1], oacc[dt][4 * g + 2], oacc[dt][4 * g + 3]};
-    red_ml[wave - 1][lane] = f32x2{m, l};
-  }
-  __syncthreads();
-  if (wave > 0) return;
-  {
-    f32x2 ml[3];
-    float mm = m;
-#pragma unroll
-    for (int w = 0; w < 3; ++w) {
-      ml[w] = red_ml[w][lane];
-      mm = fmaxf(mm, ml[w][0]);
-    }
-    const float a0 = exp2_fast(m - mm);
-    l *= a0;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) oacc[dt][i] *= a0;
-#pragma unroll
-    for (int w = 0; w < 3; ++w) {
-      const float aw = exp2_fast(ml[w][0] - mm);
-      l = __builtin_fmaf(aw, ml[w][1], l);
+    __syncthreads();  // every wave's tiles are read: the block is reused for the merge
+    // merge the four waves' (O, m, l) with the log-sum-exp rule (a wave that
+    // had no tile has m = -inf and contributes nothing); m is the same on a
+    // lane and its lane^32 partner
+    if (wave > 0) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x4 o = red_o[w][dt * 4 + g][lane];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) oacc[dt][4 * g + e] = __builtin_fmaf(aw, o[e], oacc[dt][4 * g + e]);
-        }
+        for (int g = 0; g < 4; ++g)
+          red_o[wave - 1][dt * 4 + g][lane] =
+              f32x4{oacc[dt][4 * g], oacc[dt][4 * g + 1], oacc[dt][4 * g + 2], oacc[dt][4 * g + 3]};
+      red_ml[wave - 1][lane] = f32x2{m, l};
     }
-    m = mm;
-  }
+    __syncthreads();
+    if (wave > 0) return;
+    {
+      f32x2 ml[3];
+      float mm = m;
+#pragma unroll
+      for (int w = 0; w < 3; ++w) {
+        ml[w] = red_ml[w][lane];
+        mm = fmaxf(mm, ml[w][0]);
+      }
+      const float a0 = exp2_fast(m - mm);
+      l *= a0;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) oacc[dt][i] *= a0;
+#pragma unroll
+      for (int w = 0; w < 3; ++w) {
+        const float aw = exp2_fast(ml[w][0] - mm);
+        l = __builtin_fmaf(aw, ml[w][1], l);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x4 o = red_o[w][dt * 4 + g][lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) oacc[dt][4 * g + e] = __builtin_fmaf(aw, o[e], oacc[dt][4 * g + e]);
+          }
+      }
+      m = mm;
+    }
   }
   if (row >= p.T) return;
   const float lt = sum_with_partner(l);
@@ -392,9 +390,6 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_bwd_dq_f32_kernel(A
   f32x16 dq[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) zero16(dq[dt]);
-  loads_done(qv);
-  loads_done(gv);
-  loads_done({nl2, nd});
   // dP first, then S: V's next tile is copied behind S and dQ, K's behind the next dP
   for (int kt = kt0; kt <= task.blk; kt += SPLIT) {
     const bool more = kt + SPLIT <= task.blk;
@@ -437,27 +432,27 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_bwd_dq_f32_kernel(A
     if (more) kst.stage(K, kbase, p.sk[2], (kt + SPLIT) * 32, p.T);
   }
   if constexpr (SPLIT == 4) {
-  __syncthreads();  // every wave's tiles are read: the block is reused for the sums
-  // the four waves' partial sums: waves 1-3 hand theirs to wave 0
-  if (wave > 0) {
+    __syncthreads();  // every wave's tiles are read: the block is reused for the sums
+    // the four waves' partial sums: waves 1-3 hand theirs to wave 0
+    if (wave > 0) {
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+      for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
-        red[wave - 1][dt * 4 + g][lane] = f32x4{dq[dt][4 * g], dq[dt][4 * g + 1], dq[dt][4 * g + 2], dq[dt][4 * g + 3]};
-  }
-  __syncthreads();
-  if (wave > 0) return;
+        for (int g = 0; g < 4; ++g)
+          red[wave - 1][dt * 4 + g][lane] = f32x4{dq[dt][4 * g], dq[dt][4 * g + 1], dq[dt][4 * g + 2], dq[dt][4 * g + 3]};
+    }
+    __syncthreads();
+    if (wave > 0) return;
 #pragma unroll
-  for (int w = 0; w < 3; ++w)
+    for (int w = 0; w < 3; ++w)
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+      for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 a = red[w][dt * 4 + g][lane];
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 a = red[w][dt * 4 + g][lane];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) dq[dt][4 * g + e] += a[e];
-      }
+          for (int e = 0; e < 4; ++e) dq[dt][4 * g + e] += a[e];
+        }
   }
   if (row >= p.T) return;
   float* out = fptr(p.out) + task.b * p.sout[0] + (int64_t)task.h * p.sout[1] + (int64_t)row * p.sout[2];
@@ -530,7 +525,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_bwd_dkv_f32_kernel(
   char* Qt = smem + wave * BUF;
   char* Gt = Qt + 32 * TL::RB;
   const float* vec = reinterpret_cast<const float*>(Gt + 32 * TL::RB);
-  F32Stager<D> qst, gst;
+  F32Stager<D, D <= 64> qst, gst;
   qst.init(p.sq[2], lane);
   gst.init(p.sdo[2], lane);
   const F32Tile<D> tile(l32, hh);
@@ -549,8 +544,12 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_bwd_dkv_f32_kernel(
     stage_q(wave);
     stage_g(wave);
   }
-  loads_done(kv);
-  loads_done(vv);
+  // (D = 64, 8 x 512, 16 / 4 heads: 108.5 us without, 106.3 with; at D = 32 the
+  // first tile's Q arrives before K and V, 2 x 256, 4 / 2 heads: 13.8 / 14.5)
+  if constexpr (D > 32) {
+    loads_done(kv);
+    loads_done(vv);
+  }
   for (int u = wave; u < npair; u += 4) {
     const int qt = task.blk + u / p.R;
     const bool more = u + 4 < npair;

@@ -201,22 +201,20 @@ struct Stager {
 // Copies of ROWS rows by one wave into LDS of its own (lds wave-uniform), W the
 // row width in 16-bit values, T the element type of the matrix.  A 1 KB copy is
 // RPC whole rows; its chunks differ from the first copy's by an exclusive or (the
-// swizzle's row bits of the copy and of the lane do not overlap).  Up to 4 copies
-// per 16 rows, the swizzle's period, their offsets are kept and the scalar base
-// moves for the other rows; more of them (D = 128 fp32: 8 for each of two
-// matrices) push attn_bwd_dkv_f32_kernel into scratch, whose reloads wait for the
-// copies, so there the offsets are formed at each copy and the scalar base moves
-// for every one.  fp32 forward + backward with RoPE, kept / formed, us: 2 x 1024, 16
-// / 4 heads of 128 660 / 629, 1 x 2000 1230 / 1114; of 64, 8 x 512 239 / 253, 4 x
-// 1000, 8 / 2 heads 284 / 298.  The wave waits for its copies by count
-// (copies_done), with no barrier.
-template <class T, int W, int ROWS>
+// swizzle's row bits of the copy and of the lane do not overlap).  KEPT: the
+// offsets of the copies of 16 rows, the swizzle's period, are kept and the scalar
+// base moves for the other rows.  Otherwise each is formed at its copy and the
+// scalar base moves for every one: for a kernel that has no registers left
+// (attn_bwd_dkv_f32_kernel<128>, whose 16 offsets went to scratch and whose
+// reloads waited for the copies: 367 / 309 us at 2 x 1024, 16 / 4 heads; the
+// kernels that hold them lose, attn_fwd_f32_kernel<128> 91.5 / 95.7 us there).  The
+// wave waits for its copies by count (copies_done), with no barrier.
+template <class T, int W, int ROWS, bool KEPT = true>
 struct WaveStager {
   using TL = Tile<W>;
   static constexpr int RPC = 64 / TL::NC;    // rows of a copy
   static constexpr int COPIES = ROWS / RPC;  // of a tile, whatever path it takes
   static constexpr int N = 16 / RPC;         // copies of 16 rows
-  static constexpr bool KEPT = N <= 4;
   static constexpr int EL = 16 / sizeof(T);  // elements per 16-byte chunk
   static_assert(ROWS % 16 == 0, "the swizzle's period");
   uint32_t voff[KEPT ? N : 1];  // bytes from the first row of 16; not KEPT: of the lane's row in a copy
