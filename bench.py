@@ -331,12 +331,10 @@ def time_decode(pkg, cases=DECODE_CASES, iters=50):
     (32 rollouts, Hq 8, Hkv 2, D 64, bf16 cache of `capacity` positions:
     1024 = the config's block_size, and 512 for a shorter window), through the
     C ABI with preallocated buffers, the length read from device memory as the
-    recorded decode step does: the attention (mt_gqa_attn_decode_dev: one
-    launch at these capacities) and the RoPE / cache-append kernel, each timed
-    over `iters` back-to-back launches with HIP events.  Algorithmic bytes:
-    the attention reads the group's q and L cached K and V rows once and
-    writes O; a longer cache also writes and reads one fp32 partial
-    (o, m, l) per head and 256 keys; the append reads the fp32 q / k / v
+    recorded decode step does: the attention (mt_gqa_attn_decode_dev) and the
+    RoPE / cache-append kernel, each timed over `iters` back-to-back calls with
+    HIP events.  Algorithmic bytes: the attention reads the group's q and L
+    cached K and V rows once and writes O; the append reads the fp32 q / k / v
     projections and writes q_rot and one K and one V cache row."""
     native = pkg._native
     lib = native.load()
@@ -376,9 +374,6 @@ def time_decode(pkg, cases=DECODE_CASES, iters=50):
         q_rot = torch.empty_like(q)
         ins = (ctypes.c_int64 * 6)(xq.stride(0), xq.stride(1), xk.stride(0), xk.stride(1), xv.stride(0), xv.stride(1))
         cst = (ctypes.c_int64 * 6)(*kc.stride()[:3], *vc.stride()[:3])
-        # the library's rule: one launch up to 512 keys, up to 1024 at D <= 64 with 64 (sequence, KV head) pairs
-        fused = cap <= 512 or (cap <= 1024 and d <= 64 and b * hkv >= 64)
-        ns = (L + 255) // 256
         attn = lambda: native.check(lib.mt_gqa_attn_decode_dev(  # noqa: E731
             q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), b, hq, hkv, cap, length.data_ptr(), d, st,
             scale, native.DTYPE_BF16, ws.data_ptr(), ws_bytes, sp), "mt_gqa_attn_decode_dev")
@@ -387,13 +382,11 @@ def time_decode(pkg, cases=DECODE_CASES, iters=50):
             q_rot.data_ptr(), kc.data_ptr(), vc.data_ptr(), cst, cap, b, hq, hkv, d, native.DTYPE_FP32,
             native.DTYPE_BF16, sp), "mt_decode_rope_append")
         attn_bytes = 2 * b * hkv * L * d * 2 + 2 * b * hq * d * 2
-        if not fused:
-            attn_bytes += 2 * b * hq * ns * (d + 4) * 4
         us = timed(attn, iters)
         us_app = timed(append, iters)
         app_bytes = b * (hq + 2 * hkv) * d * 4 + b * (hq + 2 * hkv) * d * 2 + d * 4
         res[f"cap{cap}_L{L}"] = {
-            "attention_kernels": "attn_decode_kernel" if fused else "attn_decode_kernel + attn_decode_combine_kernel",
+            "attention_kernels": "attn_decode_kernel (+ attn_decode_combine_kernel for a cache split over workgroups)",
             "attention_us": round(us, 2), "attention_bytes": attn_bytes,
             "attention_GBps": round(attn_bytes / (us * 1e-6) / 1e9, 1),
             "rope_append_us": round(us_app, 2), "rope_append_bytes": app_bytes}

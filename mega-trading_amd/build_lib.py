@@ -5,10 +5,11 @@ Run as ``python mega-trading_amd/build_lib.py`` or through
 travel with the source tree (they are git-ignored, not installed anywhere).
 
 * libmt_attn.so: the gfx950 kernels and their C ABI (hipcc).
-* libmt_torch.so: the PyTorch-ROCm side of the attention ops -- the GPU
-  implementations of the ``mega_trading_amd::*`` ops whose schemas, shapes
-  and autograd ``attention.py`` declares -- built with the host compiler
-  against torch's headers and linked to libmt_attn.so; no device code.
+* libmt_torch.so: the PyTorch-ROCm side of the ops -- the GPU
+  implementations and the autograd of the ``mega_trading_amd::*`` ops whose
+  schemas and shapes ``attention.py``, ``ops.py`` and ``projection.py`` declare
+  -- built with the host compiler against torch's headers and linked to
+  libmt_attn.so; no device code.
 * libmt_probe.so: a sustained-MFMA-rate probe that bench.py reports beside
   the roofline; it is not part of the attention ABI.
 """

@@ -1272,14 +1272,14 @@ __device__ __forceinline__ void dq_split_body(const AttnParams& p, int L, char* 
 }
 
 // ===========================================================================
-// Backward, dQ for D = 128: 8 waves of 32 query rows per workgroup
+// Backward, dQ for D = 128: waves of 32 query rows
 // ===========================================================================
-// As for the D = 128 forward: the 4 (head, 64-row block) pairs of a RowTask
-// split into two 32-row waves, two waves per SIMD and no spills.  At D = 128
-// attn_bwd_dq_kernel re-reads the K / V operands for each 32-query half
-// anyway, so the narrower wave costs no extra LDS reads per MFMA.  It runs
-// before the dK/dV pass (separate launches) and writes the -delta and
-// -LSE log2(e) vectors that pass reads.
+// As for the D = 128 forward: the (head, 64-row block) pairs of a RowTask (2 with
+// 4 waves a workgroup, kDq128Waves) split into two 32-row waves, two waves per SIMD
+// and no spills.  At D = 128 attn_bwd_dq_kernel re-reads the K / V operands for
+// each 32-query half anyway, so the narrower wave costs no extra LDS reads per
+// MFMA.  It runs before the dK/dV pass (separate launches) and writes the -delta
+// and -LSE log2(e) vectors that pass reads.
 template <class E, int D, bool MASK>
 __device__ __forceinline__ void dq32_tile(const char* K, const char* Vr, const typename E::v8* qop,
                                           const typename E::v8* gop, f32x16* dqacc, float lse2, float dlt, int rbase,

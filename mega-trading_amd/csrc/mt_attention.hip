@@ -184,9 +184,9 @@ void set_pairs(mt::AttnParams& p, int pairs) {
 // Waves per D = 128 dQ workgroup: 4, two workgroups per CU, so that a barrier
 // stalls half of a CU's waves and a small grid spreads over twice the CUs.
 // Against 8 waves (one workgroup per CU), forward + backward: 2 x 500, 32 / 8
-// heads 89.9 -> 80.4 us, 13 x 888, 4 / 4 heads 110.0 -> 107.9, 8 x 2048, 32 / 8
-// heads 1.460 -> 1.452 ms (the dQ kernel gains 7 %, the dK/dV kernel behind it
-// runs at a lower clock).
+// heads 89.9 -> 80.4 us, 13 x 888, 4 / 4 heads 110.0 -> 107.9.  The full grid of 8 x
+// 2048, 32 / 8 heads gains nothing (1.44-1.47 ms with either: the dQ kernel is 7 %
+// faster, the dK/dV kernel behind it runs at a lower clock).
 constexpr int kDq128Waves = 4;
 
 // Waves per D = 128 forward workgroup: 8 with 128-key K / V tiles (one
