@@ -136,7 +136,8 @@ def test_wave_private_and_split_copies_have_their_wait_states(tmp_path):
 
 
 def test_fp32_kernels_use_no_scratch(tmp_path):
-    """A spill in the fp32 loops would be reloaded between the copies in flight, each reload waiting for all of them."""
+    """A spill in the fp32 loops would be reloaded between the copies in flight, each reload waiting for all of them.
+    Every instantiation's copies have their wait states too, with kept offsets and with formed ones."""
     hipcc = _hipcc()
     if hipcc is None:
         pytest.skip("hipcc not available")
@@ -151,3 +152,4 @@ def test_fp32_kernels_use_no_scratch(tmp_path):
     assert proc.returncode == 0, proc.stderr[-2000:]
     sizes = re.findall(r"; ScratchSize: (\d+)", out.read_text())
     assert len(sizes) == 18 and set(sizes) == {"0"}
+    test_every_lds_copy_has_its_wait_states(_instructions(out.read_text()))

@@ -417,3 +417,23 @@ def test_decode_append_attention_takes_misaligned_tensors(which, dev):
     got = attn.decode_append_attention(q, k, v, cos, sin, at, n, k1, v1, repeats=hq // hkv)
     ref = attn.decode_attention(attn.decode_rope_append(q, k, v, cos, sin, at, k2, v2), k2, v2, n, repeats=hq // hkv)
     assert torch.equal(k1, k2) and torch.equal(v1, v2) and torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("dev", [False, True])
+def test_compiled_decode_step_equals_the_eager_one(dev):
+    """One functionalized graph that writes the caches: values and caches of the eager step, three steps in a row."""
+    attn = importlib.import_module("mega-trading_amd.attention")
+    b, hq, hkv, d, cap = 3, 8, 2, 64, 48
+    g = torch.Generator(device="cuda").manual_seed(21)
+    rope = model_mod.RotaryEmbedding(d, cap, theta=10_000.0).cuda()
+    k1, v1 = (torch.randn(b, hkv, cap, d, generator=g, device="cuda").bfloat16() for _ in range(2))
+    k2, v2 = k1.clone(), v1.clone()
+    torch._dynamo.reset()
+    step = torch.compile(attn.decode_append_attention, fullgraph=True, backend="aot_eager")
+    for pos in (17, 18, 19):
+        q, k, v = (torch.randn(b, n, 1, d, generator=g, device="cuda") for n in (hq, hkv, hkv))
+        at, n = ((torch.tensor([x], dtype=torch.int32, device="cuda") for x in (pos, pos + 1)) if dev else (pos, pos + 1))
+        with torch.no_grad():
+            got = step(q, k, v, rope.cos, rope.sin, at, n, k1, v1, repeats=hq // hkv)
+            ref = attn.decode_append_attention(q, k, v, rope.cos, rope.sin, at, n, k2, v2, repeats=hq // hkv)
+        assert torch.equal(got, ref) and torch.equal(k1, k2) and torch.equal(v1, v2), pos

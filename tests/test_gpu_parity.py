@@ -373,7 +373,7 @@ def test_padded_head_dim_keeps_the_query_layout(mta):
 @pytest.mark.parametrize("rope", [False, True])
 def test_fp32_tile_edges_and_both_forward_forms(b, t, hq, hkv, d, rope):
     """fp32 kernels against float64: ragged tiles, waves without a tile, and grids on both sides of the
-    row-block-per-wave rule (2048 row blocks on a 256-CU GPU).  A value is a sum of at most t + d products
+    row-block-per-wave rule (512 to 1280 row blocks on a 256-CU GPU, by the sequence's length).  A value is a sum of at most t + d products
     of values of the inputs' scale (1), each rounded to 2^-24: the error is at most (t + d) 2^-24 of that scale
     or of the result where that is larger (at t = 1 dQ and dK cancel to 0); 3e-5 at the largest size here."""
     g = torch.Generator(device="cuda").manual_seed(t * 100 + d)
