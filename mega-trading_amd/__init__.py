@@ -17,10 +17,15 @@ name carries a hyphen).  Public API:
   8-layer train step on synthetic Zipf tokens (the tokens/sec benchmark).
 """
 
-from . import model, ops, workload
+from . import _native, model, ops, workload
 from .attention import SUPPORTED_HEAD_DIMS, attention, attention_forward, decode_attention, rope_attention
 from .ops import add_rms_norm, rms_norm, swiglu_gate
 
 __all__ = ["attention", "rope_attention", "attention_forward", "decode_attention", "SUPPORTED_HEAD_DIMS",
            "rms_norm", "add_rms_norm",
            "swiglu_gate", "model", "ops", "workload"]
+
+# The ops' GPU kernels and autograd are in the library: a program that calls the
+# ops themselves (an exported one, loaded from a file) has them from the import on.
+if _native.built():
+    _native.load()

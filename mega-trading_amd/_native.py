@@ -119,6 +119,11 @@ def torch_ops_path() -> str:
     return TORCH_OPS_PATH
 
 
+def built() -> bool:
+    """Whether both libraries are there for a torch that can load them."""
+    return torch.version.hip is not None and os.path.exists(LIB_PATH) and os.path.exists(TORCH_OPS_PATH)
+
+
 def load() -> ctypes.CDLL:
     """Load libmt_attn.so (once) and declare the C signatures; also load
     libmt_torch.so, which registers the ops' GPU kernels and autograd with torch."""

@@ -6,6 +6,10 @@ gradients without an error.
 
 from __future__ import annotations
 
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -163,3 +167,18 @@ def test_a_call_whose_tables_alone_require_a_gradient_is_recorded(ops, name):
     out = getattr(ops, name)(*args)[0]
     assert out.requires_grad
     assert torch.autograd.grad(out, cos, torch.ones_like(out), allow_unused=True) == (None,)
+
+
+def test_the_ops_have_their_autograd_from_the_import_on():
+    """As an exported program calls them: no function of the package first."""
+    code = """
+import importlib, torch
+importlib.import_module("mega-trading_amd")
+x, w = (torch.empty(s, device="meta", requires_grad=True) for s in ((4, 16), (16,)))
+y, _rstd = torch.ops.mega_trading_amd.rms_norm_fwd(x, w, 1e-5)
+dx, dw = torch.autograd.grad(y, (x, w), torch.ones_like(y))
+assert dx.shape == x.shape and dw.shape == w.shape
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    proc = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=300)
+    assert proc.returncode == 0, proc.stderr[-2000:]
